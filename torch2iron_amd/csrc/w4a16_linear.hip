@@ -681,6 +681,9 @@ using t2i_host::aligned16;
 using t2i_host::fail;
 using t2i_host::LinearPlan;
 using t2i_host::plan_linear;
+using t2i_host::plan_prompt;
+using t2i_host::PROMPT_ROWS;
+using t2i_host::PromptPlan;
 
 template <int MT, int LW, int W, int CK, bool NORM, bool XROWS, bool TILED, int PRE = 0, bool NXT = false>
 hipError_t launch_t(const LinearParams& p, dim3 grid, hipStream_t s) {
@@ -754,20 +757,14 @@ hipError_t launch_plan(const LinearPlan& pl, const LinearParams& p, bool norm, b
 }
 
 // The prompt GEMM over p's rows, with its own row sums or p.xs in p.xs_parts parts.
-hipError_t launch_gemm(const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
+hipError_t launch_gemm(const PromptPlan& pl, const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
+  if (pl.kind == PromptPlan::RING) return t2i_host::launch_prompt_ring(pl, p, pp, s);
+  if (pl.kind != PromptPlan::TILES64) return hipErrorInvalidValue;
   const unsigned tiles = (unsigned)((p.M + GM_BM - 1) / GM_BM) * (unsigned)(p.N / GM_BN);
   if (!p.xs) hipLaunchKernelGGL(w4a16_gemm_kernel<0>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
   else if (p.xs_parts == 1) hipLaunchKernelGGL(w4a16_gemm_kernel<1>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
   else hipLaunchKernelGGL(w4a16_gemm_kernel<2>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
   return hipGetLastError();
-}
-
-// Rows from which the LDS-tiled GEMM replaces the 16-row-tile kernel.
-int gemm_min_rows() {
-#ifdef T2I_TUNING
-  if (const char* env = getenv("T2I_GEMM_MIN_M")) return atoi(env);
-#endif
-  return 512;
 }
 
 int check_weights(const int32_t* qweight, const int32_t* qzeros, const uint16_t* scales,
@@ -835,12 +832,14 @@ int run_linear(int epi, const uint16_t* x, int M, const uint16_t* gamma, float e
     if ((ss_in && !aligned16(ss_in)) || (g_next && !aligned16(g_next)) || (xg && !aligned16(xg)) ||
         (ss_out && ((uintptr_t)ss_out & 3u)))
       return fail(T2I_ERR_ALIGN, "chained-norm buffers: 16-byte aligned (ss_out 4-byte)");
-    if (M >= gemm_min_rows()) return fail(T2I_ERR_SHAPE, "M=%d: the chained norm serves fewer than %d rows", M, gemm_min_rows());
+    if (M >= PROMPT_ROWS) return fail(T2I_ERR_SHAPE, "M=%d: the chained norm serves fewer than %d rows", M, PROMPT_ROWS);
   }
-  if (!gamma && M >= gemm_min_rows() && N % GM_BN == 0) {
-    // prompt-sized: the LDS-tiled GEMM, over the AutoGPTQ words
+  const PromptPlan prompt = gamma || chain ? PromptPlan{PromptPlan::NONE, {0, 0, 0, 0}} : plan_prompt(M, K, N);
+  if (prompt.kind != PromptPlan::NONE && (M >= PROMPT_ROWS || (qweight && !ys))) {
+    // the LDS-tiled GEMMs, over the AutoGPTQ words (without them, fewer rows than a prompt
+    // batch's read the tiles below)
     if (!qweight)
-      return fail(T2I_ERR_SHAPE, "M=%d: prompt rows (>= %d) read qweight, which is NULL", M, gemm_min_rows());
+      return fail(T2I_ERR_SHAPE, "M=%d: prompt rows (>= %d) read qweight, which is NULL", M, PROMPT_ROWS);
     LinearParams p{};
     p.x = x;
     p.qw = reinterpret_cast<const uint32_t*>(qweight);
@@ -853,15 +852,15 @@ int run_linear(int epi, const uint16_t* x, int M, const uint16_t* gamma, float e
     p.ldx = K;
     p.ldy = paired ? N / 2 : N;
     p.epi = epi;
-    p.xs = xs;
+    p.xs = M >= PROMPT_ROWS ? xs : nullptr;   // (sums are read for a prompt batch only)
     p.xs_parts = xs_parts;
     p.ldxs = M;
     p.ys = ys;
     p.ldys = M;
-    return t2i_host::hip_status(launch_gemm(p, QkvPrepParams{}, reinterpret_cast<hipStream_t>(stream)),
+    return t2i_host::hip_status(launch_gemm(prompt, p, QkvPrepParams{}, reinterpret_cast<hipStream_t>(stream)),
                                 "w4a16 gemm launch");
   }
-  if (ys) return fail(T2I_ERR_SHAPE, "y_sums needs the prompt GEMM (M >= %d, N a multiple of %d)", gemm_min_rows(), GM_BN);
+  if (ys) return fail(T2I_ERR_SHAPE, "y_sums needs the prompt GEMM (M >= %d, N a multiple of %d)", PROMPT_ROWS, GM_BN);
   const LinearPlan pl = plan_linear(M, K, N, paired, gamma != nullptr, false);
   if (chain && !(pl.MT == 1 && pl.W == 8 && pl.CK == 4 && pl.LW <= (chain == 2 ? 1 : 2)))
     return fail(T2I_ERR_SHAPE, "M=%d K=%d N=%d: no chained-norm form of this plan", M, K, N);
@@ -905,8 +904,8 @@ int run_prefill_qkv(const uint16_t* x, const float* x_sums, int32_t B, int32_t T
   if (B < 1 || T < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv || Hq + 2 * Hkv > 0x3FFF)
     return fail(T2I_ERR_SHAPE, "B=%d T=%d Hq=%d Hkv=%d invalid", B, T, Hq, Hkv);
   const long long M = (long long)B * T;
-  if (M < gemm_min_rows() || M > T2I_MAX_ROWS)
-    return fail(T2I_ERR_SHAPE, "B*T=%lld must be in [%d, %d] (the prompt GEMM)", M, gemm_min_rows(), T2I_MAX_ROWS);
+  if (M < PROMPT_ROWS || M > T2I_MAX_ROWS)
+    return fail(T2I_ERR_SHAPE, "B*T=%lld must be in [%d, %d] (the prompt GEMM)", M, PROMPT_ROWS, T2I_MAX_ROWS);
   if (p0 < 0 || ctx_cap < 1 || p0 + T > ctx_cap)
     return fail(T2I_ERR_SHAPE, "positions %d..%d exceed the cache (%d)", p0, p0 + T - 1, ctx_cap);
   if (rope_style != 0 && rope_style != 1) return fail(T2I_ERR_VALUE, "rope_style must be 0 or 1");
@@ -933,7 +932,7 @@ int run_prefill_qkv(const uint16_t* x, const float* x_sums, int32_t B, int32_t T
   p.xs = x_sums;
   p.xs_parts = 1;
   p.ldxs = p.M;
-  return t2i_host::hip_status(launch_gemm(p, pp, reinterpret_cast<hipStream_t>(stream)), "prefill projection launch");
+  return t2i_host::hip_status(launch_gemm(plan_prompt(p.M, K, N), p, pp, reinterpret_cast<hipStream_t>(stream)), "prefill projection launch");
 }
 }  // namespace
 
@@ -1062,7 +1061,7 @@ extern "C" int t2i_w4a16_linear_tiles_chain(const uint16_t* x, int32_t M, const 
 }
 
 extern "C" int t2i_w4a16_chain_supported(int32_t M, int32_t K, int32_t N, int32_t role) {
-  if (M < 1 || M >= gemm_min_rows() || K <= 0 || K % GS || N <= 0 || N % 16) return 0;
+  if (M < 1 || M >= PROMPT_ROWS || K <= 0 || K % GS || N <= 0 || N % 16) return 0;
   const bool paired = role == 2;
   if (role < 0 || role > 2 || (paired && N % 32)) return 0;
   if (role >= 1 && K != 1024 && K != 2048) return 0;
