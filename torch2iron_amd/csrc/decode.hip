@@ -135,6 +135,8 @@ struct AttnParams {
   float eps, scale;
 };
 
+// More splits than this are merged by a kernel of their own (decode_attention_merge_kernel).
+constexpr int ATT_MERGE_CHAIN = 32;
 
 // One workgroup per (sequence b, kv head h, chunk of 16 * ROWS context slots).
 // A single workgroup per (b, h) streaming the whole context was measured 2-4x
@@ -163,7 +165,8 @@ struct AttnParams {
 //   PREP = false (t2i_decode_attention_prepared): q, k and v come normalised and
 //   rotated already, as three row arrays: qkv_ = q [B, Hq*D], qn_ = k [B, Hkv*D],
 //   kn_ = v [B, Hkv*D]; no norm weights and no RoPE table are read.
-template <int Q, int ROWS, bool PREP = true>
+//   LONG: more than ATT_MERGE_CHAIN splits; the states are left to the merge kernel.
+template <int Q, int ROWS, bool PREP = true, bool LONG = false>
 __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const int32_t* pos_, const uint16_t* qkv_,
                                                                        uint16_t* kc_, uint16_t* vc_,
                                                                        const uint16_t* qn_, const uint16_t* kn_,
@@ -486,7 +489,7 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const int
     for (int idx = tid; idx < Q * D; idx += ATT_THREADS)
       p.out[(size_t)b * p.Hq * D + (size_t)h * Q * D + idx] = 0;
   }
-  if (p.splits == 1) return;
+  if (LONG || p.splits == 1) return;
 
   // ---- 3. the last chunk of (b, h) to arrive merges every chunk's state, in chunk order ----
   // Hand-off between workgroups on different XCDs (each XCD has its own L2), at the
@@ -554,6 +557,68 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const int
         lsum > 0.0f ? (uint16_t)f32_to_bf16(o / lsum) : (uint16_t)0;
   }
   if (tid == 0) __hip_atomic_store(p.arrivals + bh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The merge of many chunk states: one workgroup per (sequence, kv head, q head) and 32
+// outputs, thread (slice sl, col): states sl, sl + 32, ... of outputs 4 col .. 4 col + 3, eight
+// in flight; the slices' states then meet in LDS, in slice order.  The last chunk to arrive
+// would read every state by itself, eight a round trip (32768 slots, 4 q heads a kv head: 470
+// states, 59 round trips, 120 of a call's 149 us; with the whole workgroup on it and 16 in
+// flight still 55 us, one CU's coherent reads of 1 MB), where a second launch costs some 3 us
+// (149 -> 33 us a call, of which the cache's 123 MB take 24 us at a large copy's rate); at 32
+// states the chain's four round trips are cheaper than the launch.
+constexpr int ATT_MERGE_DIMS = 32;
+__global__ __launch_bounds__(256) void decode_attention_merge_kernel(const float* __restrict__ part_ml,
+                                                                     const float* __restrict__ part_o,
+                                                                     uint16_t* __restrict__ out, int splits, int Q) {
+  constexpr int D = ATT_D, COLS = ATT_MERGE_DIMS / 4, SL = 256 / COLS;
+  const int bh = blockIdx.x / Q, j = blockIdx.x - bh * Q, d0 = blockIdx.y * ATT_MERGE_DIMS;
+  const int col = threadIdx.x % COLS, sl = threadIdx.x / COLS;
+  float M = -INFINITY, lsum = 0.0f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = sl; s0 < splits; s0 += 8 * SL) {
+    float ms[8], ls[8];
+    f32x4 os[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {   // unconditional loads (clamped)
+      const size_t st = ((size_t)bh * splits + min(s0 + u * SL, splits - 1)) * Q + j;
+      ms[u] = part_ml[st * 2];
+      ls[u] = part_ml[st * 2 + 1];
+      os[u] = *reinterpret_cast<const f32x4*>(part_o + st * D + d0 + 4 * col);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (ls[u] > 0.0f && s0 + u * SL < splits) {   // an empty chunk stored no context
+        const float mn = fmaxf(M, ms[u]);
+        const float fa = state_weight(M, mn), fb = exp2_fast(ms[u] - mn);
+        lsum = lsum * fa + ls[u] * fb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = o[i] * fa + os[u][i] * fb;
+        M = mn;
+      }
+    }
+  }
+  __shared__ float s_m[SL], s_l[SL];
+  __shared__ __align__(16) float s_o[SL][ATT_MERGE_DIMS];
+  *reinterpret_cast<f32x4*>(&s_o[sl][4 * col]) = o;
+  if (col == 0) {
+    s_m[sl] = M;
+    s_l[sl] = lsum;
+  }
+  __syncthreads();
+  if (threadIdx.x < ATT_MERGE_DIMS) {
+    float mx = s_m[0];
+#pragma unroll
+    for (int k = 1; k < SL; ++k) mx = fmaxf(mx, s_m[k]);
+    float l = 0.0f, v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < SL; ++k) {
+      const float f = state_weight(s_m[k], mx);
+      l = fmaf(s_l[k], f, l);
+      v = fmaf(s_o[k][threadIdx.x], f, v);
+    }
+    out[(size_t)blockIdx.x * D + d0 + threadIdx.x] = l > 0.0f ? (uint16_t)f32_to_bf16(v / l) : (uint16_t)0;
+  }
 }
 
 // ============================================================================
@@ -920,8 +985,17 @@ template <int Q, int ROWS, bool PREP>
 hipError_t launch_attention(const AttnParams& p, dim3 grid, hipStream_t s) {
   const int heads = p.Hq | p.Hkv << 15 | p.style << 30;
   const int cap_chunk = (int)((unsigned)p.ctx_cap | (unsigned)p.chunk << 23);
-  hipLaunchKernelGGL((decode_attention_kernel<Q, ROWS, PREP>), grid, dim3(ATT_THREADS), 0, s, p.pos, p.qkv, p.kc,
+  if (p.splits <= ATT_MERGE_CHAIN) {
+    hipLaunchKernelGGL((decode_attention_kernel<Q, ROWS, PREP>), grid, dim3(ATT_THREADS), 0, s, p.pos, p.qkv, p.kc,
+                       p.vc, p.qn, p.kn, heads, cap_chunk, p);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((decode_attention_kernel<Q, ROWS, PREP, true>), grid, dim3(ATT_THREADS), 0, s, p.pos, p.qkv, p.kc,
                      p.vc, p.qn, p.kn, heads, cap_chunk, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(decode_attention_merge_kernel, dim3(grid.x * Q, ATT_D / ATT_MERGE_DIMS), dim3(256), 0, s,
+                     p.part_ml, p.part_o, p.out, p.splits, Q);
   return hipGetLastError();
 }
 
