@@ -298,6 +298,223 @@ __global__ __launch_bounds__(256, 3) void prefill_attention_kernel(const Prefill
   }
 }
 
+// The max over the four lanes c, c + 16, c + 32, c + 48 of a row, in all of them: two lane
+// swaps on the VALU in place of two exchanges through LDS.
+__device__ __forceinline__ float row4_max(float v) {
+  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+// The same product with two sets of 16 query rows a wave (128 rows a workgroup).  With one
+// set a wave reads the whole K and V block (32 KB) for 16 rows: 1024 cycles of LDS a block
+// for a workgroup against 512 of MFMA.  With two, every read feeds two MFMAs and the
+// softmax (16 exponentials a lane, set and block, at a quarter rate) bounds it.  Two block
+// buffers (one barrier a block), two workgroups a CU; each lane sums its own keys' weights
+// and the four sums of a row meet after the last block; the outputs are rescaled only when a
+// row of the wave has a new max.  1999 rows from 6001 on, 32 q / 8 kv heads: 398 -> 300 us
+// (764 TFLOP/s); 16 x 250 rows from 500 on: 88 -> 71 us; 16 x 512 from 0, 16 / 8: 47.8 -> 44 us.
+template <int Q>
+__global__ __launch_bounds__(256, 2) void prefill_attention_wide_kernel(const PrefillAttnParams p) {
+  constexpr int D = PF_D;
+  constexpr int R = 2;                      // row sets a wave
+  constexpr int BQ = PF_ROWS * R / Q;       // prompt rows per q head in the tile
+  // Query blocks are dealt last block first (grid.y counts down): the causal
+  // work of a block grows with its position, so the longest go out first and
+  // the short ones fill the tail.
+  const int t0 = (gridDim.y - 1 - blockIdx.y) * BQ;
+  const int h = blockIdx.x % p.Hkv;
+  const int b = blockIdx.x / p.Hkv;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15;
+  const int r = lane >> 4;
+
+  __shared__ __align__(16) uint16_t s_k[2][PF_KEYS * PF_KLD];   // [key][dim]
+  __shared__ __align__(16) uint16_t s_vt[2][D * PF_VLD];        // [dim][key]
+
+  // ---- this lane's query row j = 16 (R wave + rs) + c of each set, as the B operand (dims 32 ks + 8 r ..) ----
+  int t_row[R], head[R], qpos[R], qmin[R];   // keys beyond qpos are masked; qmin: the set's smallest (wave-uniform)
+  u32x4 qb[R][4];
+#pragma unroll
+  for (int rs = 0; rs < R; ++rs) {
+    const int j0 = (wave * R + rs) * 16, jrow = j0 + c;
+    t_row[rs] = t0 + jrow % BQ;
+    head[rs] = h * Q + jrow / BQ;
+    qpos[rs] = p.p0 + t_row[rs];
+    // rows j0 .. j0 + 15 of the tile are prompt rows t0 + j % BQ
+    qmin[rs] = p.p0 + t0 + ((j0 % BQ) + 16 <= BQ ? j0 % BQ : 0);
+    const uint16_t* src = p.q + (((size_t)b * p.Hq + head[rs]) * p.T + min(t_row[rs], p.T - 1)) * D + 8 * r;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qb[rs][ks] = *reinterpret_cast<const u32x4*>(src + ks * 32);
+  }
+  const int last_t = min(t0 + BQ, p.T) - 1;
+  const int kend = p.p0 + last_t + 1;        // keys [0, kend) can be attended
+  const size_t cache_base = ((size_t)b * p.Hkv + h) * (size_t)p.cap * D;
+
+  float m[R], l[R];                          // l: of this lane's keys
+  f32x4 o[R][8];
+#pragma unroll
+  for (int rs = 0; rs < R; ++rs) {
+    m[rs] = -INFINITY;
+    l[rs] = 0.0f;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) o[rs][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // K / V block staging: 64 keys x 128 dims each = 1024 chunks of 16 bytes; 4 per
+  // thread.  K chunk q: key q / 16, dims 8 (q % 16), stored as loaded.  V: thread
+  // (key group g = tid % 16, octet o = tid / 16) loads keys 4 g .. 4 g + 3 of dims
+  // 8 o .. 8 o + 7 and stores each dim's four keys as one 8-byte piece of s_vt (16
+  // lanes of a store cover one dim's 64 keys: no bank conflicts).  Loads are
+  // unconditional (keys past kend reload key kend - 1: finite values whose
+  // softmax weights are zero).
+  const int vgrp = tid & 15, voct = tid >> 4;
+  auto load_block = [&](int kb, u32x4 (&kr)[4], u32x4 (&vr)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q16 = tid + 256 * u;
+      const int kkey = min(kb * PF_KEYS + (q16 >> 4), kend - 1);
+      const int vkey = min(kb * PF_KEYS + 4 * vgrp + u, kend - 1);
+      kr[u] = *reinterpret_cast<const u32x4*>(p.kc + cache_base + (size_t)kkey * D + 8 * (q16 & 15));
+      vr[u] = *reinterpret_cast<const u32x4*>(p.vc + cache_base + (size_t)vkey * D + 8 * voct);
+    }
+  };
+  auto store_block = [&](int buf, u32x4 (&kr)[4], u32x4 (&vr)[4]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q16 = tid + 256 * u;
+      *reinterpret_cast<u32x4*>(s_k[buf] + (q16 >> 4) * PF_KLD + 8 * (q16 & 15)) = kr[u];
+    }
+    const uint32_t w0[4] = {vr[0].x, vr[0].y, vr[0].z, vr[0].w};
+    const uint32_t w1[4] = {vr[1].x, vr[1].y, vr[1].z, vr[1].w};
+    const uint32_t w2[4] = {vr[2].x, vr[2].y, vr[2].z, vr[2].w};
+    const uint32_t w3[4] = {vr[3].x, vr[3].y, vr[3].z, vr[3].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // dims 2 e (low halves) and 2 e + 1 (high halves) of keys 4 g .. 4 g + 3
+      const u32x2 lo = u32x2{__builtin_amdgcn_perm(w1[e], w0[e], 0x05040100u), __builtin_amdgcn_perm(w3[e], w2[e], 0x05040100u)};
+      const u32x2 hi = u32x2{__builtin_amdgcn_perm(w1[e], w0[e], 0x07060302u), __builtin_amdgcn_perm(w3[e], w2[e], 0x07060302u)};
+      *reinterpret_cast<u32x2*>(s_vt[buf] + (8 * voct + 2 * e) * PF_VLD + 4 * vgrp) = lo;
+      *reinterpret_cast<u32x2*>(s_vt[buf] + (8 * voct + 2 * e + 1) * PF_VLD + 4 * vgrp) = hi;
+    }
+  };
+
+  const int nblocks = (kend + PF_KEYS - 1) / PF_KEYS;
+  u32x4 kr[4], vr[4];
+  load_block(0, kr, vr);
+  store_block(0, kr, vr);
+  if (nblocks > 1) load_block(1, kr, vr);
+  __syncthreads();
+  for (int kb = 0; kb < nblocks; ++kb) {
+    const uint16_t* const bk = s_k[kb & 1];
+    const uint16_t* const bv = s_vt[kb & 1];
+    // ---- S^T = K Q^T: 4 key tiles of 16 ----
+    f32x4 s[R][4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+      for (int rs = 0; rs < R; ++rs) s[rs][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const u32x4 ka = *reinterpret_cast<const u32x4*>(bk + (n * 16 + c) * PF_KLD + ks * 32 + 8 * r);
+#pragma unroll
+        for (int rs = 0; rs < R; ++rs)
+          s[rs][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka),
+                                                             __builtin_bit_cast(bf16x8, qb[rs][ks]), s[rs][n], 0, 0, 0);
+      }
+    }
+    uint32_t pw[R][4][2];                     // bf16 weights, two keys a word
+#pragma unroll
+    for (int rs = 0; rs < R; ++rs) {
+      // ---- online softmax of the lane's row (log2 domain), causal mask ----
+      // Blocks that every row of the set sees whole skip the mask.  The scale goes
+      // into the exponent's FMA (the max of the scaled scores is the scaled max); a
+      // masked score is -inf, whose weight 2^-inf is 0.
+      if (kb * PF_KEYS + PF_KEYS - 1 > qmin[rs]) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb * PF_KEYS + n * 16 + 4 * r + i > qpos[rs]) s[rs][n][i] = -INFINITY;
+      }
+      float mx = fmaxf(fmaxf(s[rs][0][0], s[rs][0][1]), fmaxf(s[rs][0][2], s[rs][0][3]));
+#pragma unroll
+      for (int n = 1; n < 4; ++n)
+        mx = fmaxf(mx, fmaxf(fmaxf(s[rs][n][0], s[rs][n][1]), fmaxf(s[rs][n][2], s[rs][n][3])));
+      const float mn = fmaxf(m[rs], row4_max(mx) * p.scale_log2);   // finite: every row attends key 0
+      if (__any(mn > m[rs])) {                // else every factor is 1
+        const float f = __builtin_amdgcn_exp2f(m[rs] - mn);         // 0 while m is -inf
+        l[rs] *= f;
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[rs][n][i] *= f;
+        m[rs] = mn;
+      }
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const uint32_t w = pack_bf16x2(__builtin_amdgcn_exp2f(fmaf(s[rs][n][i], p.scale_log2, -mn)),
+                                         __builtin_amdgcn_exp2f(fmaf(s[rs][n][i + 1], p.scale_log2, -mn)));
+          pw[rs][n][i / 2] = w;
+          l[rs] = dot2_bf16(w, 0x3F803F80u, l[rs]);   // the rounded weights
+        }
+    }
+    // ---- O^T += V^T P^T: 2 k-steps of 32 keys, 8 dim tiles ----
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        const uint16_t* vrow = bv + (n * 16 + c) * PF_VLD + ks * 32 + 4 * r;
+        const u32x2 v0 = *reinterpret_cast<const u32x2*>(vrow);
+        const u32x2 v1 = *reinterpret_cast<const u32x2*>(vrow + 16);
+        const u32x4 va = u32x4{v0.x, v0.y, v1.x, v1.y};
+#pragma unroll
+        for (int rs = 0; rs < R; ++rs) {
+          const u32x4 pb = u32x4{pw[rs][2 * ks][0], pw[rs][2 * ks][1], pw[rs][2 * ks + 1][0], pw[rs][2 * ks + 1][1]};
+          o[rs][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va),
+                                                             __builtin_bit_cast(bf16x8, pb), o[rs][n], 0, 0, 0);
+        }
+      }
+    }
+    // the next block into the other buffer (its last reader passed the barrier before this block)
+    if (kb + 1 < nblocks) {
+      store_block((kb + 1) & 1, kr, vr);
+      if (kb + 2 < nblocks) load_block(kb + 2, kr, vr);
+      __syncthreads();
+    }
+  }
+
+  // ---- normalise and store: the lane holds row jrow's dims 16 n + 4 r .. + 3 ----
+#pragma unroll
+  for (int rs = 0; rs < R; ++rs) {
+    float lt = l[rs];                          // the row's four lanes (all lanes take part)
+    lt += __shfl_xor(lt, 16, 64);
+    lt += __shfl_xor(lt, 32, 64);
+    if (t_row[rs] >= p.T) continue;            // uniform over the four lanes of a row
+    uint16_t* dst = p.out + ((size_t)b * p.T + t_row[rs]) * p.Hq * D + (size_t)head[rs] * D + 4 * r;
+    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+    float hs = 0.0f;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const float y0 = round_bf16(o[rs][n][0] * inv), y1 = round_bf16(o[rs][n][1] * inv);
+      const float y2 = round_bf16(o[rs][n][2] * inv), y3 = round_bf16(o[rs][n][3] * inv);
+      *reinterpret_cast<u32x2*>(dst + n * 16) = u32x2{pack_bf16x2(y0, y1), pack_bf16x2(y2, y3)};
+      hs += ((y0 + y1) + (y2 + y3));
+    }
+    if (p.out_sums) {
+      // the head's 128 values are one quantisation group of the next product's k
+      hs += __shfl_xor(hs, 16, 64);
+      hs += __shfl_xor(hs, 32, 64);
+      if (r == 0) p.out_sums[(size_t)head[rs] * p.B * p.T + (size_t)b * p.T + t_row[rs]] = hs;
+    }
+  }
+}
+
 }  // namespace t2i
 
 // ============================================================================
@@ -344,15 +561,26 @@ int run_prefill_attention(const uint16_t* q, int32_t B, int32_t T, int32_t p0, i
   p.q = q; p.kc = k_cache; p.vc = v_cache; p.out = out; p.out_sums = out_sums;
   p.B = B; p.T = T; p.Hq = Hq; p.Hkv = Hkv; p.cap = ctx_cap; p.p0 = p0;
   p.scale_log2 = (float)(1.4426950408889634 / sqrt((double)D));
-  const int bq = t2i::PF_ROWS / Q;
+  // The wide form where its blocks of 128 rows make at least 400 of the longest one's length
+  // (a block's work grows from p0 to p0 + T keys): with fewer the longest block is the call
+  // (2000 rows from 0, 256 blocks: 61 us against 53; 2048 rows of 8 q heads a kv head from 0,
+  // 512 blocks: 70 against 67; 1999 rows from 6001, 504 blocks: 300 against 398).
+  const int bq2 = 2 * t2i::PF_ROWS / Q;
+  const long long blocks2 = (long long)B * Hkv * ((T + bq2 - 1) / bq2);
+  const bool wide = (double)blocks2 * (2.0 * p0 + T) >= 800.0 * ((double)p0 + T);
+  const int bq = wide ? bq2 : t2i::PF_ROWS / Q;
   const dim3 grid(B * Hkv, (T + bq - 1) / bq);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+#define T2I_PREFILL(q)                                                                                      \
+  if (wide) hipLaunchKernelGGL((t2i::prefill_attention_wide_kernel<q>), grid, dim3(256), 0, s, p);          \
+  else hipLaunchKernelGGL((t2i::prefill_attention_kernel<q>), grid, dim3(256), 0, s, p)
   switch (Q) {
-    case 1: hipLaunchKernelGGL((t2i::prefill_attention_kernel<1>), grid, dim3(256), 0, s, p); break;
-    case 2: hipLaunchKernelGGL((t2i::prefill_attention_kernel<2>), grid, dim3(256), 0, s, p); break;
-    case 4: hipLaunchKernelGGL((t2i::prefill_attention_kernel<4>), grid, dim3(256), 0, s, p); break;
-    default: hipLaunchKernelGGL((t2i::prefill_attention_kernel<8>), grid, dim3(256), 0, s, p); break;
+    case 1: T2I_PREFILL(1); break;
+    case 2: T2I_PREFILL(2); break;
+    case 4: T2I_PREFILL(4); break;
+    default: T2I_PREFILL(8); break;
   }
+#undef T2I_PREFILL
   return t2i_host::hip_status(hipGetLastError(), "prefill attention launch");
 }
 }  // namespace
