@@ -122,8 +122,9 @@ int t2i_w4a16_rmsnorm_gate_up(const uint16_t* x, int32_t M, const uint16_t* norm
  * kernels, same arithmetic, bit-identical outputs.  qweight (may be NULL) is the
  * AutoGPTQ original: given, the call also serves prompt rows (M >= 512 without
  * the fused norm, which read qweight) and reads qweight for the few decode plans
- * that read it faster; NULL: every plan reads the tiles, and prompt rows are
- * rejected (T2I_ERR_SHAPE).  epilogue:
+ * that read it faster and for 65 to 511 rows where the prompt GEMM is faster; NULL:
+ * every plan reads the tiles (65 to 511 rows then add in another order), and prompt
+ * rows are rejected (T2I_ERR_SHAPE).  epilogue:
  * T2I_TILES_STORE (y0 = y, or y0 = bf16(bf16(y) + residual) with residual != NULL),
  * T2I_TILES_SWIGLU (paired weight, y0 = h) or T2I_TILES_PAIRED (y0 = gate, y1 = up).
  * norm_weight != NULL: the fused RMSNorm (no residual).

@@ -1,5 +1,7 @@
 // W4A16 group-128 linear for gfx950: y[M, N] = x[M, K] . W^T (M = 1: GEMV;
-// M <= 64: batched decode; more rows: a prompt batch, 16-row tiles in grid.z).
+// M <= 64: batched decode).  More rows with qweight at hand run a prompt GEMM
+// (plan_prompt: the ring kernel of w4a16_gemm.hip or the 64 x 128 kernel below),
+// except where the plan finds this kernel faster (16-row tiles in grid.z).
 //
 // Weights stay in the AutoGPTQ layout.  One int32 word of qweight holds the
 // 8 consecutive k of one column, which is exactly the 8 bf16 values one lane
