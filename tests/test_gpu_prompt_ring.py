@@ -25,6 +25,12 @@ SHAPES = [
     ("64x128, 2 slices", 520, 2176, 128), ("64x128, 2 slices", 577, 2048, 384), ("64x128, 2 slices", 300, 1024, 6144),
     ("64x128, pairs", 2050, 2176, 1024), ("64x128, pairs", 197, 2048, 12288),
     ("128x256", 390, 1920, 12288), ("128x256", 321, 2176, 12288), ("128x256", 3969, 3072, 2048),
+    # few steps, two to five: the prologue's loads reach past the last one, and every load that is
+    # off is then waited beside one that is on
+    ("64x128, pairs", 500, 256, 8192), ("64x128, pairs", 257, 384, 12288), ("64x128, pairs", 321, 512, 8192),
+    ("128x256", 321, 256, 20480), ("128x256", 450, 384, 10752), ("128x256", 257, 512, 16384),
+    ("64x128, 2 slices", 500, 384, 4096), ("64x128, 2 slices", 197, 512, 8192), ("64x128, 2 slices", 390, 640, 4096),
+    ("64x128, 2 slices", 321, 896, 4096), ("32x64, 4 slices", 116, 1920, 4096), ("32x64, 4 slices", 113, 2176, 3968),
 ]
 
 

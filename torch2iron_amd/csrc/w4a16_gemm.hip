@@ -6,8 +6,8 @@
 // columns, a lane NJ consecutive columns (so pairs meet in a lane and results are stored
 // from registers).  A step is one quantisation group (128 of K).
 //   * Every operand of a step comes by loads into LDS, three tiles deep (a step's tile is
-//     requested two steps ahead, its words three), counted by hand: no wait in the loop ever
-//     finds a load in flight that it needs.
+//     requested two steps ahead, its words three), counted by hand: a step ends when all but
+//     its last requests, the words three steps ahead, have landed.
 //   * A packed word becomes eight bf16 (144 + q - z): nibbles to bytes, 16 - z added to all
 //     four bytes of a half, then each pair under the exponent byte 0x43: eleven VALU
 //     instructions.  The bias is the same for every column, so the zero-point correction is
@@ -119,8 +119,9 @@ __device__ __forceinline__ i32x4 tile_rsrc(const void* p) {
 // One 16-byte (dma4: 4-byte) piece a lane into LDS at lds + 16 (4) lane, written as asm so
 // that the compiler's own waits (it waits for every load into LDS before any LDS read)
 // leave it in flight; dma_wait covers it.  M0 takes the LDS address, with one wait state
-// before the load.  lanes: all (~0) or none (0: nothing is read or written, the load still
-// counts for dma_wait); every call is made by whole waves, so all lanes are on again after it.
+// before the load.  lanes: all (~0) or none (0: nothing is read or written, and nothing is
+// assumed of when such a load counts or leaves the count: waits past one wait for everything);
+// every call is made by whole waves, so all lanes are on again after it.
 __device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t off, uint32_t soff, uint32_t lds, uint64_t lanes) {
   asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b64 exec, -1"
                :: "s"(lds), "v"(off), "s"(rsrc), "s"(soff), "s"(lanes) : "memory", "m0");
@@ -307,7 +308,8 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   for (int i = 0; i < S::OPS_S; ++i) load_s(2, 2, 1, i);
 #pragma unroll
   for (int q = 0; q < S::OPS_W; ++q) load_w(2, 2, q);
-  dma_wait<S::OPS + S::OPS_S + S::OPS_W>();
+  if (loads > 2) dma_wait<S::OPS + S::OPS_S + S::OPS_W>();
+  else dma_wait<0>();          // (steps 2 and on are switched off)
   __syncthreads();
   if constexpr (XSP > 0) {
     given_xs(0, 0);
@@ -334,7 +336,8 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
 #pragma unroll
       for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(B0[ks][j]));
   }
-  dma_wait<S::OPS_W>();        // behind it: step 2's words
+  if (loads > 2) dma_wait<S::OPS_W>();   // behind it: step 2's words
+  else dma_wait<0>();
   __syncthreads();             // (slot 0's words are consumed: step 0 loads step 3's there)
 
   // The first AHEAD k-steps' fragments are read before the step, its last fragment's sums are
@@ -438,7 +441,10 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) scp[j] = sc[j];
-    dma_wait<S::OPS_W>();    // tile s + 2 has landed; step s + 3's words may be on their way
+    // Tile s + 2 has landed; step s + 3's words may be on their way, unless they are switched
+    // off: then the last loads that are on are waited for whatever the others count.
+    if (s + 3 < loads) dma_wait<S::OPS_W>();
+    else dma_wait<0>();
     __syncthreads();
   };
   {
