@@ -81,6 +81,17 @@ def test_paired_and_swiglu(gpu, form, m, k, n):
     assert (h == chain).float().mean() > 0.99
 
 
+@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES])
+def test_equal_rows_give_equal_bits(gpu, form, m, k, n):
+    """A row's result does not depend on its place in the call (nor on who sums the row)."""
+    w, x = _weight(k, n, m + k, gpu), _x(1, k, m + n, gpu).expand(m, k).contiguous()
+    y = ops.linear(x, w)
+    assert torch.equal(y, y[:1].expand(m, n)), form
+    if m >= ops.PROMPT_GEMM_ROWS:
+        y = ops.linear(x, w, x_sums=x.float().view(m, -1, 128).sum(-1).t().contiguous())
+        assert torch.equal(y, y[:1].expand(m, n)), form
+
+
 @pytest.mark.parametrize("form,m,k,n", [s for s in SHAPES if s[1] >= ops.PROMPT_GEMM_ROWS],
                          ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES if m >= ops.PROMPT_GEMM_ROWS])
 @pytest.mark.parametrize("parts", [1, 2])

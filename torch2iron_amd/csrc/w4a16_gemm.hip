@@ -13,8 +13,11 @@
 //     instructions.  The bias is the same for every column, so the zero-point correction is
 //     -144 x the row's sum over the group, which is where the accumulators start: one FMA
 //     per output and group (total += scale * acc) instead of two.  A wave sums the rows of
-//     its own fragments of the next tile with MFMAs against bf16 -144 (or takes given sums),
-//     so each row is summed once a workgroup and not once a wave.
+//     one fragment of the next tile with MFMAs against bf16 -144 (or takes given sums), so
+//     each row is summed once a workgroup and not once a wave.  It begins its steps with that
+//     fragment, whose sums it still holds; the others' come through LDS behind the step's
+//     barrier.  So every accumulator starts at its row sums: equal rows give equal bits
+//     wherever they stand in the call.
 //   * Step s + 1's words are unpacked beside step s's MFMAs, the previous fragment's sums
 //     are folded beside the next one's, loads go out one every few MFMAs.  The order is the
 //     program's (empty asm ties; the compiler otherwise sinks the folds and unpacking behind
@@ -62,9 +65,9 @@ struct GemmShape {
   static constexpr int TILE = BN % ATT_D == 0 ? BM * (BN + 8) * 2 : 0;  // the bf16 tile of EPI_QKV_PREP
   static constexpr int LDS = STAGES > PART ? (STAGES > TILE ? STAGES : TILE) : (PART > TILE ? PART : TILE);
   // loads into LDS a wave issues each step
-  static constexpr int FW = MF / WN, OPS_A = 4 * FW, OPS_W = W_BYTES / 1024 / WN, OPS_S = (PIECES + WN - 1) / WN;
+  static constexpr int OPS_A = KSG, OPS_W = W_BYTES / 1024 / WN, OPS_S = (PIECES + WN - 1) / WN;
   static constexpr int OPS = OPS_A + OPS_S + OPS_W;
-  static_assert(MF % WN == 0 && (MF % WK == 0 || WK % MF == 0), "whole row fragments and pieces");
+  static_assert(MF == WN && (MF & (MF - 1)) == 0 && (MF % WK == 0 || WK % MF == 0), "a row fragment a wave, whole pieces");
   static_assert(W_BYTES % (1024 * WN) == 0 && OPS_S <= 2, "the same number of loads in every wave");
 };
 
@@ -173,17 +176,14 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   auto group_of = [&](int s) { return min(s * WK + wk, groups - 1); };
 
   // ---- loads into LDS (every offset stays inside the tensors: rows and groups are clamped) ----
-  // Activations: the wave brings row fragments wn FW .. of its slice, one MFMA A operand
+  // Activations: the wave brings row fragment wn of its slice, one MFMA A operand
   // (lane (c, r): row c, k 32 ks + 8 r ..) a load.
-  constexpr int FW = S::FW;
   const int mlim = p.M - 1 - m0;
   const i32x4 xrsrc = tile_rsrc(p.x + (size_t)m0 * p.ldx);
-  uint32_t xoff[FW][KSG];
+  uint32_t xoff[KSG];
 #pragma unroll
-  for (int f = 0; f < FW; ++f)
-#pragma unroll
-    for (int ks = 0; ks < KSG; ++ks)
-      xoff[f][ks] = (uint32_t)min(16 * (wn * FW + f) + c, mlim) * (uint32_t)(p.ldx * 2) + 16u * r + 64u * ks;
+  for (int ks = 0; ks < KSG; ++ks)
+    xoff[ks] = (uint32_t)min(16 * wn + c, mlim) * (uint32_t)(p.ldx * 2) + 16u * r + 64u * ks;
   // Packed words: 1 KB of the tile's [16][BN] a load.
   constexpr int WROWS = 256 / BN > 0 ? 256 / BN : 1;   // word rows a load covers (BN = 128: 2)
   static_assert(BN == 64 || BN == 128 || BN == 256, "whole word rows a load");
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     return (uint64_t)v << 32 | v;
   };
   auto load_a = [&](int s, int slot, int q) {
-    dma16(xrsrc, xoff[q / KSG][q % KSG], (uint32_t)group_of(s) * (GS * 2), lds_a + slot * WK * S::A_BYTES + q * 1024,
+    dma16(xrsrc, xoff[q], (uint32_t)group_of(s) * (GS * 2), lds_a + slot * WK * S::A_BYTES + q * 1024,
           lanes_of(s));
   };
   auto load_w = [&](int s, int slot, int q) {
@@ -241,9 +241,12 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   };
 
   // ---- LDS reads ----
+  // The wave takes the tile's row fragments from its own on: its fragment k is row fragment row_frag(k).
+  auto row_frag = [&](int k) { return (wn + k) & (MF - 1); };
   const uint32_t aoff = wk * S::A_BYTES + 16 * lane;
-  auto read_a = [&](int slot, int u) {
-    return *reinterpret_cast<const u32x4*>(s_a + slot * WK * S::A_BYTES + u * 1024 + aoff);
+  auto read_a = [&](int slot, int u) {   // unit u: k-step u % KSG of the wave's fragment u / KSG
+    return *reinterpret_cast<const u32x4*>(s_a + slot * WK * S::A_BYTES + row_frag(u / KSG) * (KSG * 1024) + aoff +
+                                           u % KSG * 1024);
   };
   auto read_w = [&](int slot, int ks, uint32_t (&w)[NJ]) {
     load_words<NJ>(reinterpret_cast<const uint32_t*>(s_w + (slot * WK + wk) * S::W_BYTES) + (4 * ks + r) * BN + lcol, w);
@@ -265,16 +268,23 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
       asm volatile("" : "+v"(add[j]), "+v"(sc[j]));
     }
   };
-  auto xs_at = [&](int par, int k) { return reinterpret_cast<f32x4*>(s_x + (par * WK + wk) * BM + 16 * k + 4 * r); };
-  // The wave's row fragments of a tile: -144 x the row sums, the accumulators' start.  Precomputed
-  // sums (XSP > 0): lane i takes row i.  Else MFMAs of the fragment (units a) against bf16 -144.
-  auto given_xs = [&](int par, int slot) {
-    static_assert(FW <= 4, "a lane a row");
-    const int row = 16 * FW * wn + min(lane, 16 * FW - 1);
-    const float* src = reinterpret_cast<const float*>(s_s + (slot * WK + wk) * S::S_BYTES + (S::P_SC + 1) * 256) + row;
-    float v = src[0];
-    if constexpr (XSP == 2) v += src[S::P_XS * 64];
-    if (lane < 16 * FW) s_x[(par * WK + wk) * BM + row] = -GM_BIAS * v;
+  // -144 x the row sums, the accumulators' start: of the wave's fragment k (rows 4 r .. of it) ...
+  auto xs_at = [&](int par, int k) {
+    return reinterpret_cast<f32x4*>(s_x + (par * WK + wk) * BM + 16 * row_frag(k) + 4 * r);
+  };
+  // ... and, for its first fragment, from the precomputed sums (XSP > 0), or by MFMAs of the
+  // fragment (units a) against bf16 -144.
+  auto given_xs = [&](int slot) {
+    const unsigned char* src = s_s + (slot * WK + wk) * S::S_BYTES + (S::P_SC + 1) * 256 + (16 * wn + 4 * r) * 4;
+    f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    if constexpr (XSP == 2) {
+      const f32x4 v2 = *reinterpret_cast<const f32x4*>(src + S::P_XS * 256);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += v2[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= -GM_BIAS;
+    return v;
   };
   const u32x4 mbias = {0xC310C310u, 0xC310C310u, 0xC310C310u, 0xC310C310u};   // bf16 -144
   auto sum_unit = [&](u32x4 a, f32x4 xs) {
@@ -311,17 +321,14 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   if (loads > 2) dma_wait<S::OPS + S::OPS_S + S::OPS_W>();
   else dma_wait<0>();          // (steps 2 and on are switched off)
   __syncthreads();
+  f32x4 xown = {0.f, 0.f, 0.f, 0.f};   // the start of the wave's first fragment in the step to come
   if constexpr (XSP > 0) {
-    given_xs(0, 0);
+    xown = given_xs(0);
   } else {
 #pragma unroll
-    for (int f = 0; f < FW; ++f) {
-      f32x4 xs = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KSG; ++ks) xs = sum_unit(read_a(0, (wn * FW + f) * KSG + ks), xs);
-      if (c == 0) *xs_at(0, wn * FW + f) = xs;
-    }
+    for (int ks = 0; ks < KSG; ++ks) xown = sum_unit(read_a(0, ks), xown);
   }
+  if (c == 0) *xs_at(0, 0) = xown;
   {
     uint32_t add[NJ], w[KSG][NJ];
     read_sz(0, 0, add, sc0);
@@ -344,7 +351,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   // carried into total during the next step (scp: their scales).
   constexpr int AHEAD = KSG + 2, RINGA = 2 * KSG;   // reads run this many k-steps ahead of their MFMAs
   constexpr int UNITS = KSG * MF;
-  static_assert(UNITS % RINGA == 0 && FW < MF, "the ring of fragments starts every step at its first slot");
+  static_assert(UNITS % RINGA == 0 && MF > 1, "the ring of fragments starts every step at its first slot");
   u32x4 a[RINGA];
   f32x4 P[2][NJ];
   float scp[NJ];
@@ -360,7 +367,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     constexpr int par = decltype(PAR)::value;
     constexpr int NW = KSG * NJ, SLOTS = (MF - 1) * NW;   // words a lane, MFMAs after fragment 0
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    u32x4 an[2][KSG];
+    u32x4 an[KSG];
     f32x4 xv[4], xs = zero;
     uint32_t w[KSG][NJ], addn[NJ];
     GemmUnpack un[NW];
@@ -387,21 +394,17 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
           const int e = ks * NJ + j;              // 0 .. 4 NJ - 1
-          // (fragment 0 gets its row sums afterwards: they are read after the step's barrier)
           P[k & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              av, B[ks][j], ks > 0 ? P[k & 1][j] : k == 0 ? zero : xv[k & 3], 0, 0, 0);
+              av, B[ks][j], ks > 0 ? P[k & 1][j] : k == 0 ? xown : xv[k & 3], 0, 0, 0);
           if (j == 0) {
             const int n = u + AHEAD;
-            if (k == 0 && ks == 0) {
-              xv[1] = *xs_at(par, 1);
-              xv[0] = *xs_at(par, 0);
-            }
+            if (k == 0 && ks == 0) xv[1] = *xs_at(par, 1);
             if (ks == 1 && k + 2 < MF) xv[(k + 2) & 3] = *xs_at(par, k + 2);
             if (k == 0) read_w(b1, ks, w[ks]);
-            // the next tile's row sums: the wave's fragments, each read beside one
+            // the next tile's row sums: the wave's first fragment, read beside the first
             // fragment's products, summed beside the next one's and written after them
-            if (XSP == 0 && k < FW) an[k & 1][ks] = read_a(b1, (wn * FW + k) * KSG + ks);
-            if (XSP == 0 && k >= 1 && k <= FW) xs = sum_unit(an[(k - 1) & 1][ks], ks == 0 ? zero : xs);
+            if (XSP == 0 && k == 0) an[ks] = read_a(b1, ks);
+            if (XSP == 0 && k == 1) xs = sum_unit(an[ks], ks == 0 ? zero : xs);
             a[n % RINGA] = n < UNITS ? read_a(b0, n) : read_a(b1, n - UNITS);
           } else if (j == 1) {
             // the loads, evenly over the fragments
@@ -419,7 +422,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
             for (int q = q0; q < q1; ++q) {
               const float v = P[(k + 1) & 1][q >> 2][q & 3];
               if (k == 0) fma1(MF - 1, q, v, scp);
-              else fma1(k - 1, q, k == 1 ? v + xv[0][q & 3] : v, sc);
+              else fma1(k - 1, q, v, sc);
             }
           }
           if (k > 0) {
@@ -436,8 +439,10 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
         }
       }
       if (k == 0) read_sz(s + 1, b1, addn, scn);
-      if (XSP == 0 && k >= 1 && k <= FW && c == 0) *xs_at(1 - par, wn * FW + k - 1) = xs;
-      if (XSP > 0 && k == 1) given_xs(1 - par, b1);
+      if (k == 1) {
+        xown = XSP > 0 ? given_xs(b1) : xs;
+        if (c == 0) *xs_at(1 - par, 0) = xown;
+      }
     }
 #pragma unroll
     for (int j = 0; j < NJ; ++j) scp[j] = sc[j];
@@ -473,11 +478,11 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   constexpr int MS = MF > WK ? MF / WK : 1;
   const bool stores = wk * MS < MF;   // (more slices than fragments: the last slices' waves have none)
   f32x4 out[MS][NJ];
-  int fr[MS];   // the row fragments of this wave's share
+  int fr[MS];   // the tile's row fragments of this wave's share
   if constexpr (WK == 1) {
 #pragma unroll
     for (int mi = 0; mi < MF; ++mi) {
-      fr[mi] = mi;
+      fr[mi] = row_frag(mi);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) out[mi][j] = total[mi][j];
     }
@@ -490,12 +495,13 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     __syncthreads();
 #pragma unroll
     for (int mi = 0; mi < MS; ++mi) {
-      fr[mi] = min(wk * MS + mi, MF - 1);
+      const int own = min(wk * MS + mi, MF - 1);   // of the wave's fragments
+      fr[mi] = row_frag(own);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        f32x4 v = part[((wn * MF + fr[mi]) * NJ + j) * 64 + lane];
+        f32x4 v = part[((wn * MF + own) * NJ + j) * 64 + lane];
 #pragma unroll
-        for (int k = 1; k < WK; ++k) v += part[(((k * WN + wn) * MF + fr[mi]) * NJ + j) * 64 + lane];
+        for (int k = 1; k < WK; ++k) v += part[(((k * WN + wn) * MF + own) * NJ + j) * 64 + lane];
         out[mi][j] = v;
       }
     }
