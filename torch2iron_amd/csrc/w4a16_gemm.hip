@@ -1,6 +1,6 @@
 // Prompt-sized W4A16 GEMM for gfx950: y[M, N] = x[M, K] . W^T for some tens to thousands of
 // rows, over the AutoGPTQ words.  (w4a16_linear.hip holds the 64 x 128 kernel that stays
-// where it is the faster one; plan_prompt below chooses.)
+// where it is the faster one; plan_prompt chooses.)
 //
 // A workgroup has WN waves along N and WK slices of K; a wave computes 16 MF rows x 16 NJ
 // columns, a lane NJ consecutive columns (so pairs meet in a lane and results are stored
@@ -32,15 +32,11 @@
 // graph-launched): gate_up 8192 x 2048 x 12288 620 -> 455, down 4001 x 6144 x 2048 150 -> 105,
 // 8192 x 2048 x 4096 197 -> 144, 8192 x 1024 x 4096 100 -> 86; against the decode tiles, gate_up
 // 331 x 2048 x 12288 55 -> 33.
-#include <math.h>
-#include <stdio.h>
-#include <stdlib.h>
-
-#include <algorithm>
 #include <type_traits>
 
 #include "t2i_common.h"
 #include "w4a16_tile.h"
+#include "prompt_plan.h"
 #include "qk_prep.h"
 
 namespace t2i {
@@ -639,7 +635,6 @@ using namespace t2i;
 template <int MF, int NJ, int WN, int WK>
 hipError_t launch_one(const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
   using S = GemmShape<MF, NJ, WN, WK, 0>;
-  if (p.N % S::BN) return hipErrorInvalidValue;
   const unsigned tiles = (unsigned)((p.M + S::BM - 1) / S::BM) * (unsigned)(p.N / S::BN);
   if (!p.xs) hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 0>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
   else if (p.xs_parts == 1) hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 1>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
@@ -658,66 +653,8 @@ hipError_t launch_one(const LinearParams& p, const QkvPrepParams& pp, hipStream_
 
 namespace t2i_host {
 
-// The kernel for an M x K x N product of more than 64 rows, from a fit of every form's time
-// (us; g = K / 128 groups, R rounds of the chip's 256 CUs) to a sweep of M = 65 .. 8192 over
-// the decoders' eight projection shapes, graph-launched.  Each line's constants are the fit;
-// the fits are within 15 % of the sweep and the choice within 8 % of the fastest form.
-//   decode tiles of 16 rows (fewer than 512 rows):  3.5 + 0.00085 x (16-row x 64-column tiles) x g
-//   2,2,2,4: 32 x 64, K in 4 slices (fewer than 512 rows):  2.5 + R (3.3 + 0.28 g)
-//   4,2,4,2: 64 x 128, K in 2 slices:  2.5 + R (4 + 0.66 g)
-//   4,2,4,1: 64 x 128, two workgroups a CU:  2 + 5.5 + 1.22 g a pair, 4 + 0.88 g a single
-//   8,2,8,1: 128 x 256:  3 + 6.5 + g (1.36 .. 1.8 with the round's fill) a round, and a tenth for
-//     its one workgroup a CU with the fused q|k|v epilogue (5000 rows, K = 1024: 82 against 81 us)
-//   the 64 x 128 kernel of three workgroups a CU (512 rows and more):  3 + 1.05 g, 2 + 1.65 g,
-//   2.5 + 2.3 g with one, two, three on a CU
-// The choice depends on M, K and N alone, so a projection's fused and plain forms give the
-// same bits.
-PromptPlan plan_prompt(int M, int K, int N) {
-  PromptPlan best{PromptPlan::NONE, {0, 0, 0, 0}};
-#ifdef T2I_TUNING
-  if (const char* env = getenv("T2I_PROMPT")) {
-    PromptPlan o{PromptPlan::RING, {0, 0, 0, 0}};
-    if (sscanf(env, "%d,%d,%d,%d", &o.cfg[0], &o.cfg[1], &o.cfg[2], &o.cfg[3]) == 4 &&
-        N % (16 * o.cfg[1] * o.cfg[2]) == 0)
-      return o;
-    return PromptPlan{M >= PROMPT_ROWS ? PromptPlan::TILES64 : PromptPlan::NONE, {0, 0, 0, 0}};
-  }
-#endif
-  const double g = K / 128;
-  double cost = 1e30;
-  auto offer = [&](double c, PromptPlan::Kind kind, int a, int b, int d, int e) {
-    if (c < cost) {
-      cost = c;
-      best = PromptPlan{kind, {a, b, d, e}};
-    }
-  };
-  const bool prompt = M >= PROMPT_ROWS;
-  if (M <= 64) return best;
-  if (prompt && N % 128) return best;
-  if (!prompt) offer(3.5 + 0.00085 * ((M + 15) / 16) * (N / 64.0) * g, PromptPlan::NONE, 0, 0, 0, 0);
-  const double t64 = (double)((M + 63) / 64) * (N / 128);
-  if (prompt)
-    offer(t64 <= 256 ? 3 + 1.05 * g : t64 <= 512 ? 2 + 1.65 * g : std::max(1.0, t64 / 768) * (2.5 + 2.3 * g),
-          PromptPlan::TILES64, 0, 0, 0, 0);
-  // the ring kernel addresses its tensors with 32-bit byte offsets
-  if ((double)K * N / 2 >= 4e9 || (double)M * K / 16 >= 4e9) return best;
-  if (!prompt && N % 64 == 0)
-    offer(2.5 + ceil((M + 31) / 32 * (N / 64) / 256.0) * (3.3 + 0.28 * g), PromptPlan::RING, 2, 2, 2, 4);
-  if (N % 128 == 0) {
-    const double pairs = floor(t64 / 512), rest = t64 - 512 * pairs;
-    offer(2.5 + ceil(t64 / 256) * (4 + 0.66 * g), PromptPlan::RING, 4, 2, 4, 2);
-    offer(2 + pairs * (5.5 + 1.22 * g) + (rest == 0 ? 0 : rest <= 256 ? 4 + 0.88 * g : 5.5 + 1.22 * g), PromptPlan::RING,
-          4, 2, 4, 1);
-  }
-  if (N % 256 == 0) {
-    const double t = (double)((M + 127) / 128) * (N / 256), r = ceil(t / 256);
-    offer(1.1 * (3 + (r - 1) * (6.5 + 1.8 * g) + 6.5 + g * (1.36 + 0.44 * (t - (r - 1) * 256) / 256)), PromptPlan::RING, 8,
-          2, 8, 1);
-  }
-  return best;
-}
-
 hipError_t launch_prompt_ring(const PromptPlan& pl, const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
+  if (!prompt_form_serves(pl, p.N, p.epi == EPI_QKV_PREP || p.xs || p.ys)) return hipErrorInvalidValue;
 #define T2I_PROMPT_LAUNCH(a, b, c, d) \
   if (pl.cfg[0] == a && pl.cfg[1] == b && pl.cfg[2] == c && pl.cfg[3] == d) return launch_one<a, b, c, d>(p, pp, s);
   T2I_PROMPT_CONFIGS(T2I_PROMPT_LAUNCH)

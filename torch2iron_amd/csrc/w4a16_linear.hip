@@ -33,6 +33,7 @@
 
 #include "t2i_common.h"
 #include "w4a16_tile.h"
+#include "prompt_plan.h"
 #include "qk_prep.h"
 
 namespace t2i {
@@ -761,7 +762,7 @@ hipError_t launch_plan(const LinearPlan& pl, const LinearParams& p, bool norm, b
 // The prompt GEMM over p's rows, with its own row sums or p.xs in p.xs_parts parts.
 hipError_t launch_gemm(const PromptPlan& pl, const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
   if (pl.kind == PromptPlan::RING) return t2i_host::launch_prompt_ring(pl, p, pp, s);
-  if (pl.kind != PromptPlan::TILES64) return hipErrorInvalidValue;
+  if (pl.kind != PromptPlan::TILES64 || !t2i_host::prompt_form_serves(pl, p.N, true)) return hipErrorInvalidValue;
   const unsigned tiles = (unsigned)((p.M + GM_BM - 1) / GM_BM) * (unsigned)(p.N / GM_BN);
   if (!p.xs) hipLaunchKernelGGL(w4a16_gemm_kernel<0>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
   else if (p.xs_parts == 1) hipLaunchKernelGGL(w4a16_gemm_kernel<1>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);

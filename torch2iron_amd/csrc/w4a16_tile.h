@@ -924,18 +924,8 @@ struct LinearPlan {
 // wide: the plan for 16-wave workgroups (the one-launch decode step's).
 LinearPlan plan_linear(int M, int K, int N, bool paired, bool norm, bool wide);
 
-// Rows from which a product is a prompt batch: the LDS-tiled kernels serve it whatever its
-// shape (N a multiple of 128); from 65 rows they do where they are faster.
-constexpr int PROMPT_ROWS = 512;
-
-// What runs an M x K x N product without a fused norm: the decode linear's tiles (NONE),
-// the 64 x 128 kernel (TILES64) or a form of the ring kernel (RING: row fragments a wave,
-// columns a lane, waves along N, k slices).
-struct PromptPlan {
-  enum Kind { NONE, TILES64, RING } kind;
-  int cfg[4];
-};
-PromptPlan plan_prompt(int M, int K, int N);
+// The ring kernel's form pl over p (prompt_plan.h).
+struct PromptPlan;
 hipError_t launch_prompt_ring(const PromptPlan& pl, const t2i::LinearParams& p, const t2i::QkvPrepParams& pp,
                               hipStream_t s);
 }  // namespace t2i_host
