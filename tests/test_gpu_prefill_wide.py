@@ -1,6 +1,7 @@
-"""Prompt attention where the blocks of 128 rows fill the chip (two row sets a wave), and on
-both sides of that line: one row, ragged last blocks, one key block and many, every q-head
-count a kv head, against float64 attention on the device.
+"""Prompt attention with two row sets a wave (blocks of 128 rows) and, beside it, with one: one
+row, ragged last blocks, one key block and many, every q-head count a kv head, against float64
+attention on the device.  Which of the two a case runs is checked on the host
+(test_prefill_plan).
 
 Tolerance: bf16 keeps 8 significant bits, so one rounding is up to 2^-8 of the value.  The
 weights are rounded and divided by the sum of the rounded ones: 2^-8 (sum p |v| + |o|); the
@@ -17,12 +18,15 @@ from torch2iron_amd import ops
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 
-# (B, rows, first position, kv heads, q heads a kv head); the first two lie on the two sides of the line
-CASES = [(100, 1, 0, 8, 1), (99, 1, 0, 8, 1), (20, 600, 0, 8, 1), (13, 500, 0, 8, 2), (51, 3, 500, 8, 4),
-         (9, 129, 3001, 8, 4), (26, 61, 1500, 4, 8), (60, 65, 63, 8, 2)]
+# two row sets a wave or one (csrc/prefill_plan.h), B, rows, first position, kv heads, q heads a kv head
+CASES = [(False, 100, 1, 0, 8, 1), (False, 99, 1, 0, 8, 1), (False, 20, 600, 0, 8, 1), (False, 13, 500, 0, 8, 2),
+         (False, 51, 3, 500, 8, 4), (False, 9, 129, 3001, 8, 4), (True, 26, 61, 1500, 4, 8), (False, 60, 65, 63, 8, 2),
+         (True, 52, 255, 100, 8, 1), (True, 64, 97, 100, 8, 2), (True, 64, 127, 63, 8, 2), (True, 16, 512, 0, 8, 2),
+         (True, 63, 33, 500, 8, 4), (True, 256, 15, 500, 4, 8), (False, 100, 8, 200, 4, 8)]
 
 
-@pytest.mark.parametrize("b,t,p0,hkv,q_per", CASES, ids=[f"B{c[0]}-T{c[1]}-p{c[2]}-H{c[3]}x{c[4]}" for c in CASES])
+@pytest.mark.parametrize("b,t,p0,hkv,q_per", [c[1:] for c in CASES],
+                         ids=["B%d-T%d-p%d-H%dx%d" % c[1:] for c in CASES])
 def test_prompt_attention(gpu, b, t, p0, hkv, q_per):
     d, hq, n = 128, hkv * q_per, p0 + t
     g = torch.Generator(device=gpu).manual_seed(b * 1000 + t)

@@ -15,6 +15,7 @@
 #include <math.h>
 
 #include "t2i_common.h"
+#include "prefill_plan.h"
 #include "qk_prep.h"
 
 namespace t2i {
@@ -561,14 +562,8 @@ int run_prefill_attention(const uint16_t* q, int32_t B, int32_t T, int32_t p0, i
   p.q = q; p.kc = k_cache; p.vc = v_cache; p.out = out; p.out_sums = out_sums;
   p.B = B; p.T = T; p.Hq = Hq; p.Hkv = Hkv; p.cap = ctx_cap; p.p0 = p0;
   p.scale_log2 = (float)(1.4426950408889634 / sqrt((double)D));
-  // The wide form where its blocks of 128 rows make at least 400 of the longest one's length
-  // (a block's work grows from p0 to p0 + T keys): with fewer the longest block is the call
-  // (2000 rows from 0, 256 blocks: 61 us against 53; 2048 rows of 8 q heads a kv head from 0,
-  // 512 blocks: 70 against 67; 1999 rows from 6001, 504 blocks: 300 against 398).
-  const int bq2 = 2 * t2i::PF_ROWS / Q;
-  const long long blocks2 = (long long)B * Hkv * ((T + bq2 - 1) / bq2);
-  const bool wide = (double)blocks2 * (2.0 * p0 + T) >= 800.0 * ((double)p0 + T);
-  const int bq = wide ? bq2 : t2i::PF_ROWS / Q;
+  const bool wide = t2i_host::prefill_wide(B, T, p0, Hkv, Q);
+  const int bq = (wide ? 2 : 1) * t2i::PF_ROWS / Q;
   const dim3 grid(B * Hkv, (T + bq - 1) / bq);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 #define T2I_PREFILL(q)                                                                                      \
