@@ -1,5 +1,5 @@
-"""The ring kernel of the prompt products (more than 64 rows), each of its forms at the
-edges of its tiles: ragged row tiles, one row past a tile, odd group counts (a last step
+"""The prompt products of more than 64 rows: each form of the ring kernel, and what serves the
+shapes beside them, at the edges of its tiles: ragged row tiles, one row past a tile, odd group counts (a last step
 without a partner) and group counts its k slices do not divide.
 
 Reference: float64 on the device over the exactly dequantised weights
@@ -19,19 +19,31 @@ from torch2iron_amd.formats import W4A16Weight, interleave_gate_up
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 
-# the form that plan_prompt gives the shape, rows, K, N
+# what plan_prompt (csrc/prompt_plan.h) gives the product with its own row sums, rows, K, N;
+# test_prompt_plan holds the plan to these names
 SHAPES = [
-    ("32x64, 4 slices", 500, 3200, 1024), ("32x64, 4 slices", 470, 3072, 1024),
+    ("decode tiles", 500, 3200, 1024), ("decode tiles", 470, 3072, 1024),
     ("64x128, 2 slices", 520, 2176, 128), ("64x128, 2 slices", 577, 2048, 384), ("64x128, 2 slices", 300, 1024, 6144),
-    ("64x128, pairs", 2050, 2176, 1024), ("64x128, pairs", 197, 2048, 12288),
+    ("64x128 kernel", 2050, 2176, 1024), ("64x128, pairs", 577, 1920, 6144), ("64x128, pairs", 1100, 2176, 3072),
+    ("64x128, pairs", 197, 2048, 12288),
     ("128x256", 390, 1920, 12288), ("128x256", 321, 2176, 12288), ("128x256", 3969, 3072, 2048),
     # few steps, two to five: the prologue's loads reach past the last one, and every load that is
     # off is then waited beside one that is on
     ("64x128, pairs", 500, 256, 8192), ("64x128, pairs", 257, 384, 12288), ("64x128, pairs", 321, 512, 8192),
     ("128x256", 321, 256, 20480), ("128x256", 450, 384, 10752), ("128x256", 257, 512, 16384),
-    ("64x128, 2 slices", 500, 384, 4096), ("64x128, 2 slices", 197, 512, 8192), ("64x128, 2 slices", 390, 640, 4096),
-    ("64x128, 2 slices", 321, 896, 4096), ("32x64, 4 slices", 116, 1920, 4096), ("32x64, 4 slices", 113, 2176, 3968),
+    ("64x128, pairs", 500, 384, 4096), ("64x128, 2 slices", 197, 512, 8192), ("64x128, 2 slices", 390, 640, 4096),
+    ("64x128, 2 slices", 321, 896, 4096), ("decode tiles", 116, 1920, 4096), ("decode tiles", 113, 2176, 3968),
 ]
+# the same with given row sums
+SUMS_SHAPES = [
+    ("64x128, 2 slices", 520, 2176, 128), ("64x128, 2 slices", 577, 2048, 384), ("64x128, 2 slices", 833, 2304, 1024),
+    ("64x128 kernel", 2050, 2176, 1024), ("64x128 kernel", 1100, 2176, 3072),
+    ("128x256", 3969, 3072, 2048), ("128x256", 520, 1920, 12288), ("128x256", 1153, 1024, 6144),
+]
+
+
+def _ids(shapes):
+    return [f"M{m}-K{k}-N{n}" for _, m, k, n in shapes]
 
 
 def _bound(ref):
@@ -50,7 +62,7 @@ def _x(m, k, seed, dev):
     return torch.randn(m, k, generator=torch.Generator().manual_seed(seed)).to(BF16).to(dev)
 
 
-@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES])
+@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=_ids(SHAPES))
 def test_linear_and_residual(gpu, form, m, k, n):
     w, x = _weight(k, n, m + k, gpu), _x(m, k, m + n, gpu)
     ref = _ref(x, w)
@@ -63,7 +75,7 @@ def test_linear_and_residual(gpu, form, m, k, n):
     assert torch.equal(out, (y.float() + res.float()).to(BF16))
 
 
-@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES])
+@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=_ids(SHAPES))
 def test_paired_and_swiglu(gpu, form, m, k, n):
     gate, up = ow.synthetic_tensors(k, n // 2, seed=m), ow.synthetic_tensors(k, n // 2, seed=m + 1)
     w, x = W4A16Weight.from_numpy(*interleave_gate_up(gate, up), device=gpu), _x(m, k, m + n, gpu)
@@ -81,19 +93,15 @@ def test_paired_and_swiglu(gpu, form, m, k, n):
     assert (h == chain).float().mean() > 0.99
 
 
-@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES])
+@pytest.mark.parametrize("form,m,k,n", SHAPES, ids=_ids(SHAPES))
 def test_equal_rows_give_equal_bits(gpu, form, m, k, n):
-    """A row's result does not depend on its place in the call (nor on who sums the row)."""
+    """A row's result does not depend on its place in the call."""
     w, x = _weight(k, n, m + k, gpu), _x(1, k, m + n, gpu).expand(m, k).contiguous()
     y = ops.linear(x, w)
     assert torch.equal(y, y[:1].expand(m, n)), form
-    if m >= ops.PROMPT_GEMM_ROWS:
-        y = ops.linear(x, w, x_sums=x.float().view(m, -1, 128).sum(-1).t().contiguous())
-        assert torch.equal(y, y[:1].expand(m, n)), form
 
 
-@pytest.mark.parametrize("form,m,k,n", [s for s in SHAPES if s[1] >= ops.PROMPT_GEMM_ROWS],
-                         ids=[f"M{m}-K{k}-N{n}" for _, m, k, n in SHAPES if m >= ops.PROMPT_GEMM_ROWS])
+@pytest.mark.parametrize("form,m,k,n", SUMS_SHAPES, ids=_ids(SUMS_SHAPES))
 @pytest.mark.parametrize("parts", [1, 2])
 def test_given_row_sums(gpu, form, m, k, n, parts):
     w, x = _weight(k, n, m + k, gpu), _x(m, k, m + n, gpu)
@@ -101,9 +109,12 @@ def test_given_row_sums(gpu, form, m, k, n, parts):
     ref = _ref(x, w)
     y = ops.linear(x, w, x_sums=sums, sum_parts=parts)
     assert ((y.double() - ref).abs() <= _bound(ref)).all(), form
+    x = x[:1].expand(m, k).contiguous()     # equal rows: equal bits
+    y = ops.linear(x, w, x_sums=x.float().view(m, -1, 128 // parts).sum(-1).t().contiguous(), sum_parts=parts)
+    assert torch.equal(y, y[:1].expand(m, n)), form
 
 
-@pytest.mark.parametrize("m,k,n", [(577, 2048, 384), (2050, 2176, 1024), (520, 2048, 12288)])
+@pytest.mark.parametrize("m,k,n", [(577, 2048, 384), (2050, 2176, 1024), (520, 2048, 12288), (577, 1920, 6144)])
 def test_swiglu_output_sums(gpu, m, k, n):
     """The half-group sums of h, within 1e-5 of the sum of the magnitudes (fp32, 64 terms)."""
     gate, up = ow.synthetic_tensors(k, n // 2, seed=m), ow.synthetic_tensors(k, n // 2, seed=m + 1)
@@ -116,7 +127,8 @@ def test_swiglu_output_sums(gpu, m, k, n):
 
 
 @pytest.mark.parametrize("style", [0, 1])
-@pytest.mark.parametrize("b,t,p0,hq,hkv,k", [(4, 509, 3, 16, 8, 1024), (1, 520, 0, 1, 1, 2176), (5, 133, 1, 16, 8, 2048)])
+@pytest.mark.parametrize("b,t,p0,hq,hkv,k", [(4, 509, 3, 16, 8, 1024), (1, 520, 0, 1, 1, 2176), (5, 133, 1, 16, 8, 2048),
+                                             (3, 1333, 1, 16, 8, 1024)])
 def test_fused_projection_matches_two_launches(gpu, b, t, p0, hq, hkv, k, style):
     d, cap = 128, t + p0 + 5
     w, x = _weight(k, (hq + 2 * hkv) * d, t, gpu), _x(b * t, k, t + 1, gpu)

@@ -24,73 +24,99 @@ struct PromptPlan {
   int cfg[4];
 };
 
-// Whether the plan's kernel can run a product of N columns; batch: with what only a prompt
-// batch's calls have (given row sums, output sums, the fused q|k|v epilogue), which needs
-// tiles of whole 128-column pieces.  The launchers refuse a product that fails this.
-inline bool prompt_form_serves(const PromptPlan& pl, int N, bool batch) {
-  if (pl.kind == PromptPlan::NONE) return false;
-  if (pl.kind == PromptPlan::RING && (pl.cfg[1] < 1 || pl.cfg[1] > 8 || pl.cfg[2] < 1 || pl.cfg[2] > 16)) return false;
-  const int cols = pl.kind == PromptPlan::TILES64 ? 128 : 16 * pl.cfg[1] * pl.cfg[2];
-  return N % cols == 0 && !(batch && cols % 128);
+// A kernel's time (us) as a fit, g = K / 128 groups: with up to `res` workgroups on each of the
+// 256 CUs, level o (o workgroups on the fullest CU) is one[o] = {at its start, a group, across
+// the level, a group of that}; with more it is many = {fixed, a group, a round of 256 res, a
+// group of that, the last round's idle share, a group of that}.
+struct PromptFit {
+  int rows, cols, res;
+  double one[3][4], many[6];
+  double us(int M, int K, int N) const {
+    const double t = (double)((M + rows - 1) / rows) * (N / cols), g = K / 128, slots = 256.0 * res;
+    if (t <= slots) {
+      const int o = std::max(1, (int)ceil(t / 256)) - 1;
+      const double share = t / 256 - o;
+      return one[o][0] + one[o][1] * g + share * (one[o][2] + one[o][3] * g);
+    }
+    const double r = t / slots, idle = ceil(r) - r;
+    return many[0] + many[1] * g + r * (many[2] + many[3] * g) + idle * (many[4] + many[5] * g);
+  }
+};
+
+// The ring kernel's forms: 64 x 128 tiles (two workgroups a CU), 64 x 128 with K in two slices,
+// 128 x 256 (its estimate is the least sure, 5 to 95 % of the fit -7 to +8 %: it is taken from
+// 3 % on).  One fit serves own and given row sums, which differ by 1 %; with given ones the
+// first form is nowhere the fastest, and is not built for them.
+struct PromptForm {
+  int cfg[4];
+  PromptFit fit;
+  double over;
+  bool given;
+};
+constexpr PromptForm PROMPT_FORMS[] = {
+    {{4, 2, 4, 1}, {64, 128, 2, {{5.25, 0.8, 0.17, 0.06}, {4.86, 1.28, 1.3, 0.07}}, {1.77, 0.22, 4.61, 1.22, 2.79, 0.47}}, 1.0, false},
+    {{4, 2, 4, 2}, {64, 128, 1, {{5.56, 0.56, -0.45, 0.17}}, {0.44, 0.15, 4.73, 0.62, 4.49, 0.51}}, 1.0, true},
+    {{8, 2, 8, 1}, {128, 256, 1, {{8.28, 1.51, 2.43, 0.27}}, {1.98, 0.31, 9.43, 1.7, 5.67, 1.16}}, 1.03, true},
+};
+// The 64 x 128 kernel, with its own row sums and with given ones (which save it a third of its
+// MFMAs).
+constexpr PromptFit TILES64_FIT[2] = {
+    {64, 128, 3, {{-1.64, 1.1, 2.95, 0.02}, {4.55, 1.29, 0.23, 0.2}, {6.01, 1.83, -0.96, 0.37}},
+     {4.46, 0.02, 2.37, 2.05, -1.16, 0.4}},
+    {64, 128, 3, {{-2.09, 1.08, 3.39, -0.02}, {4.35, 1.21, 1.11, 0.07}, {6.5, 1.66, -0.76, 0.24}},
+     {5.92, -0.1, 2.15, 1.84, -1.71, 0.49}},
+};
+
+// Whether the plan's kernel exists and can run a product of N columns, on given row sums or its
+// own.  The launchers refuse a product that fails this (columns past the last whole tile would
+// stay unwritten).
+inline bool prompt_form_serves(const PromptPlan& pl, int N, bool sums) {
+  if (pl.kind == PromptPlan::TILES64) return N % 128 == 0;
+  if (pl.kind == PromptPlan::RING)
+    for (const PromptForm& f : PROMPT_FORMS)
+      if (std::equal(f.cfg, f.cfg + 4, pl.cfg)) return N % f.fit.cols == 0 && (f.given || !sums);
+  return false;
 }
 
-// The kernel for an M x K x N product of more than 64 rows, from a fit of every form's time
-// (us; g = K / 128 groups, R rounds of the chip's 256 CUs) to a sweep of M = 65 .. 8192 over
-// the decoders' eight projection shapes, graph-launched.  Each line's constants are the fit;
-// the fits are within 15 % of the sweep and the choice within 8 % of the fastest form.
-//   decode tiles of 16 rows (fewer than 512 rows):  3.5 + 0.00085 x (16-row x 64-column tiles) x g
-//   2,2,2,4: 32 x 64, K in 4 slices (fewer than 512 rows):  2.5 + R (3.3 + 0.28 g)
-//   4,2,4,2: 64 x 128, K in 2 slices:  2.5 + R (4 + 0.66 g)
-//   4,2,4,1: 64 x 128, two workgroups a CU:  2 + 5.5 + 1.22 g a pair, 4 + 0.88 g a single
-//   8,2,8,1: 128 x 256:  3 + 6.5 + g (1.36 .. 1.8 with the round's fill) a round, and a tenth for
-//     its one workgroup a CU with the fused q|k|v epilogue (5000 rows, K = 1024: 82 against 81 us)
-//   the 64 x 128 kernel of three workgroups a CU (512 rows and more):  3 + 1.05 g, 2 + 1.65 g,
-//   2.5 + 2.3 g with one, two, three on a CU
-// The choice depends on M, K and N alone, so a projection's fused and plain forms give the
-// same bits.
-inline PromptPlan plan_prompt(int M, int K, int N) {
+// The kernel for an M x K x N product of more than 64 rows: the one of the least estimated time.
+// Fits and choice are from a sweep of M = 65 .. 8192 over the decoders' eight projection shapes,
+// every kernel graph-launched on both kinds of row sums and behind the fused q|k|v epilogue (572
+// measured choices): the fits are within 4 to 8 % of nine times in ten, the choice is within 8 %
+// of the fastest (11 % at 1024 x 2048 -> 12288), and 3 choices are 3 to 4 % slower than the
+// kernel that served the product before the ring kernel came.  The decode tiles (fewer than 512
+// rows) are 1.5 + 1 + 0.143 g a round of 256 workgroups of 16 rows x 64 columns.  A form of 32 x
+// 64 tiles with K in four slices was measured nowhere faster by more than 0.2 %.
+// sums: the rows' sums are given.  The choice depends on M, K, N and that alone, so a
+// projection's fused and plain forms give the same bits.  Products of two to four groups lie
+// outside the sweep: no ring launch was measured under 8.5 us (K = 256: 173 rows -> 5120 7.7 on
+// the decode tiles, 8.9 on the ring; 410 -> 6144 17.0, 9.9).
+inline PromptPlan plan_prompt(int M, int K, int N, bool sums) {
   PromptPlan best{PromptPlan::NONE, {0, 0, 0, 0}};
-  const double g = K / 128;
-  double cost = 1e30;
-  auto offer = [&](double c, PromptPlan::Kind kind, int a, int b, int d, int e) {
-    if (c < cost) {
-      cost = c;
-      best = PromptPlan{kind, {a, b, d, e}};
-    }
-  };
   const bool prompt = M >= PROMPT_ROWS;
-  if (M <= 64) return best;
-  if (prompt && N % 128) return best;
+  if (M <= 64 || N % 128) return best;
   // the ring kernel addresses its tensors with 32-bit byte offsets
   const bool ring = (double)K * N / 2 < 4e9 && (double)M * K / 16 < 4e9;
+  if (prompt) best.kind = PromptPlan::TILES64;
 #ifdef T2I_TUNING
   // a form for every product that it can serve, the 64 x 128 kernel or the decode tiles for the rest
   if (const char* env = getenv("T2I_PROMPT")) {
     PromptPlan o{PromptPlan::RING, {0, 0, 0, 0}};
     if (ring && sscanf(env, "%d,%d,%d,%d", &o.cfg[0], &o.cfg[1], &o.cfg[2], &o.cfg[3]) == 4 &&
-        prompt_form_serves(o, N, false))
+        prompt_form_serves(o, N, sums))
       return o;
-    return PromptPlan{prompt ? PromptPlan::TILES64 : PromptPlan::NONE, {0, 0, 0, 0}};
+    return best;
   }
 #endif
-  if (!prompt) offer(3.5 + 0.00085 * ((M + 15) / 16) * (N / 64.0) * g, PromptPlan::NONE, 0, 0, 0, 0);
-  const double t64 = (double)((M + 63) / 64) * (N / 128);
-  if (prompt)
-    offer(t64 <= 256 ? 3 + 1.05 * g : t64 <= 512 ? 2 + 1.65 * g : std::max(1.0, t64 / 768) * (2.5 + 2.3 * g),
-          PromptPlan::TILES64, 0, 0, 0, 0);
   if (!ring) return best;
-  if (!prompt && N % 64 == 0)
-    offer(2.5 + ceil((M + 31) / 32 * (N / 64) / 256.0) * (3.3 + 0.28 * g), PromptPlan::RING, 2, 2, 2, 4);
-  if (N % 128 == 0) {
-    const double pairs = floor(t64 / 512), rest = t64 - 512 * pairs;
-    offer(2.5 + ceil(t64 / 256) * (4 + 0.66 * g), PromptPlan::RING, 4, 2, 4, 2);
-    offer(2 + pairs * (5.5 + 1.22 * g) + (rest == 0 ? 0 : rest <= 256 ? 4 + 0.88 * g : 5.5 + 1.22 * g), PromptPlan::RING,
-          4, 2, 4, 1);
-  }
-  if (N % 256 == 0) {
-    const double t = (double)((M + 127) / 128) * (N / 256), r = ceil(t / 256);
-    offer(1.1 * (3 + (r - 1) * (6.5 + 1.8 * g) + 6.5 + g * (1.36 + 0.44 * (t - (r - 1) * 256) / 256)), PromptPlan::RING, 8,
-          2, 8, 1);
+  const double g = K / 128;
+  double least = prompt ? TILES64_FIT[sums].us(M, K, N) : 1.5 + ceil((M + 15) / 16 * (N / 64.0) / 256) * (1 + 0.143 * g);
+  for (const PromptForm& f : PROMPT_FORMS) {
+    if (!prompt_form_serves({PromptPlan::RING, {f.cfg[0], f.cfg[1], f.cfg[2], f.cfg[3]}}, N, sums)) continue;
+    const double us = f.over * std::max(8.5, f.fit.us(M, K, N));
+    if (us < least) {
+      least = us;
+      best = PromptPlan{PromptPlan::RING, {f.cfg[0], f.cfg[1], f.cfg[2], f.cfg[3]}};
+    }
   }
   return best;
 }

@@ -52,18 +52,19 @@ struct GemmShape {
   static constexpr int A_BYTES = BM * GS * 2;            // one slice's activation tile
   static constexpr int W_BYTES = GS / 8 * BN * 4;        // and its packed words
   // its scales, zero words and precomputed row sums, in pieces of 256 bytes
-  static constexpr int P_SC = BN > 128 ? BN / 128 : 1, P_Z = 1, P_XS = BM > 64 ? BM / 64 : 1;
+  static constexpr int P_SC = BN / 128, P_Z = 1, P_XS = BM > 64 ? BM / 64 : 1;
   static constexpr int PIECES = P_SC + P_Z + XSP * P_XS;
   static constexpr int S_BYTES = PIECES * 256;
   static constexpr int X_BYTES = 2 * BM * 4;             // -144 x the row sums, two steps
   static constexpr int STAGES = WK * (GM_RING * (A_BYTES + W_BYTES + S_BYTES) + X_BYTES);
   static constexpr int PART = WK > 1 ? WAVES * MF * NJ * 1024 : 0;      // the slices' partial sums
-  static constexpr int TILE = BN % ATT_D == 0 ? BM * (BN + 8) * 2 : 0;  // the bf16 tile of EPI_QKV_PREP
+  static constexpr int TILE = BM * (BN + 8) * 2;                        // the bf16 tile of EPI_QKV_PREP
   static constexpr int LDS = STAGES > PART ? (STAGES > TILE ? STAGES : TILE) : (PART > TILE ? PART : TILE);
   // loads into LDS a wave issues each step
   static constexpr int OPS_A = KSG, OPS_W = W_BYTES / 1024 / WN, OPS_S = (PIECES + WN - 1) / WN;
   static constexpr int OPS = OPS_A + OPS_S + OPS_W;
-  static_assert(MF == WN && (MF & (MF - 1)) == 0 && (MF % WK == 0 || WK % MF == 0), "a row fragment a wave, whole pieces");
+  static_assert(MF == WN && (MF & (MF - 1)) == 0 && MF % WK == 0, "a row fragment a wave, whole pieces");
+  static_assert(BN % 128 == 0 && ATT_D == 128, "whole heads and half groups of output sums a tile");
   static_assert(W_BYTES % (1024 * WN) == 0 && OPS_S <= 2, "the same number of loads in every wave");
 };
 
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   for (int ks = 0; ks < KSG; ++ks)
     xoff[ks] = (uint32_t)min(16 * wn + c, mlim) * (uint32_t)(p.ldx * 2) + 16u * r + 64u * ks;
   // Packed words: 1 KB of the tile's [16][BN] a load.
-  constexpr int WROWS = 256 / BN > 0 ? 256 / BN : 1;   // word rows a load covers (BN = 128: 2)
-  static_assert(BN == 64 || BN == 128 || BN == 256, "whole word rows a load");
+  constexpr int WROWS = 256 / BN;   // word rows a load covers (BN = 128: 2)
+  static_assert(BN == 128 || BN == 256, "whole word rows a load");
   const i32x4 wrsrc = tile_rsrc(p.qw + n0);
   const uint32_t woff = (uint32_t)(wn * S::OPS_W * WROWS + lane / (64 / WROWS)) * (uint32_t)(p.N * 4) + 16u * (lane % (64 / WROWS));
   // Pieces of scales, zeros and row sums: piece wn + WN i of the slice (past the last: the first again).
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     if (piece < S::P_SC) {
       src = reinterpret_cast<const unsigned char*>(p.sc + n0 + 128 * piece);
       pstride[i] = (uint32_t)p.N * 2;
-      poff[i] = 4u * min(lane, BN / 2 - 1);
+      poff[i] = 4u * lane;
     } else if (!is_xs[i]) {
       src = reinterpret_cast<const unsigned char*>(p.qz + (n0 >> 3));
       pstride[i] = (uint32_t)(p.N >> 3) * 4;
@@ -471,8 +472,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
 
   // ---- the slices' sums meet in LDS, in slice order; wave (wn, wk) keeps row
   // fragments wk MF / WK .. of its columns ----
-  constexpr int MS = MF > WK ? MF / WK : 1;
-  const bool stores = wk * MS < MF;   // (more slices than fragments: the last slices' waves have none)
+  constexpr int MS = MF / WK;
   f32x4 out[MS][NJ];
   int fr[MS];   // the tile's row fragments of this wave's share
   if constexpr (WK == 1) {
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
     __syncthreads();
 #pragma unroll
     for (int mi = 0; mi < MS; ++mi) {
-      const int own = min(wk * MS + mi, MF - 1);   // of the wave's fragments
+      const int own = wk * MS + mi;   // of the wave's fragments
       fr[mi] = row_frag(own);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
@@ -505,49 +505,46 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   }
 
   if (p.epi == EPI_QKV_PREP) {
-    if constexpr (BN % ATT_D == 0) {
-      // The tile is BN / 128 heads of rows m0 ..: parked as bf16, then each 16-lane
-      // row takes head vectors through prep_vector, as prefill_prep_kernel does.
-      constexpr int LD = BN + 8;
-      uint16_t* const tile = reinterpret_cast<uint16_t*>(smem);
+    // The tile is BN / 128 heads of rows m0 ..: parked as bf16, then each 16-lane
+    // row takes head vectors through prep_vector, as prefill_prep_kernel does.
+    constexpr int LD = BN + 8;
+    uint16_t* const tile = reinterpret_cast<uint16_t*>(smem);
 #pragma unroll
-      for (int mi = 0; mi < MS; ++mi)
+    for (int mi = 0; mi < MS; ++mi)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (!stores) continue;
-          uint32_t* dst = reinterpret_cast<uint32_t*>(tile + (16 * fr[mi] + 4 * r + i) * LD + wn * 16 * NJ + NJ * c);
+      for (int i = 0; i < 4; ++i) {
+        uint32_t* dst = reinterpret_cast<uint32_t*>(tile + (16 * fr[mi] + 4 * r + i) * LD + wn * 16 * NJ + NJ * c);
 #pragma unroll
-          for (int j = 0; j < NJ / 2; ++j) dst[j] = pack_bf16x2(out[mi][2 * j][i], out[mi][2 * j + 1][i]);
-        }
-      // The RoPE rows come first, all of them: one wait, behind the barrier, and not one a
-      // vector.
-      constexpr int HEADS = BN / ATT_D, VECS = BM * HEADS / (4 * S::WAVES);
-      static_assert(VECS * 4 * S::WAVES == BM * HEADS, "whole rounds of head vectors");
-      u32x4 rp[VECS];
-      int tt[VECS], bb[VECS];
-#pragma unroll
-      for (int i = 0; i < VECS; ++i) {
-        const int m = min(m0 + (4 * wave + r + 4 * S::WAVES * i) / HEADS, p.M - 1);
-        bb[i] = m / pp.T;
-        tt[i] = m - bb[i] * pp.T;
-        rp[i] = *reinterpret_cast<const u32x4*>(pp.rope + (size_t)(pp.p0 + tt[i]) * ATT_D + 8 * c);
+        for (int j = 0; j < NJ / 2; ++j) dst[j] = pack_bf16x2(out[mi][2 * j][i], out[mi][2 * j + 1][i]);
       }
-      const u32x4 gq = prep_load(pp.qn, c, pp.style), gk = prep_load(pp.kn, c, pp.style);
-      __syncthreads();
+    // The RoPE rows come first, all of them: one wait, behind the barrier, and not one a
+    // vector.
+    constexpr int HEADS = BN / ATT_D, VECS = BM * HEADS / (4 * S::WAVES);
+    static_assert(VECS * 4 * S::WAVES == BM * HEADS, "whole rounds of head vectors");
+    u32x4 rp[VECS];
+    int tt[VECS], bb[VECS];
 #pragma unroll
-      for (int i = 0; i < VECS; ++i) {
-        const int v = 4 * wave + r + 4 * S::WAVES * i, row = v / HEADS, hh = v % HEADS;
-        if (m0 + row >= p.M) continue;   // uniform over the 16-lane row
-        const int head = n0 / ATT_D + hh;
-        const bool isq = head < pp.Hq, normed = head < pp.Hq + pp.Hkv;
-        const u32x4 raw = prep_load(tile + row * LD + hh * ATT_D, c, pp.style);
-        const u32x4 y = prep_vector(raw, rp[i], isq ? gq : gk, normed, pp.style, pp.eps);
-        uint16_t* dst;
-        if (isq) dst = pp.q + (((size_t)bb[i] * pp.Hq + head) * pp.T + tt[i]) * ATT_D;
-        else if (normed) dst = pp.kc + (((size_t)bb[i] * pp.Hkv + (head - pp.Hq)) * pp.cap + pp.p0 + tt[i]) * ATT_D;
-        else dst = pp.vc + (((size_t)bb[i] * pp.Hkv + (head - pp.Hq - pp.Hkv)) * pp.cap + pp.p0 + tt[i]) * ATT_D;
-        prep_store(dst, c, pp.style, y);
-      }
+    for (int i = 0; i < VECS; ++i) {
+      const int m = min(m0 + (4 * wave + r + 4 * S::WAVES * i) / HEADS, p.M - 1);
+      bb[i] = m / pp.T;
+      tt[i] = m - bb[i] * pp.T;
+      rp[i] = *reinterpret_cast<const u32x4*>(pp.rope + (size_t)(pp.p0 + tt[i]) * ATT_D + 8 * c);
+    }
+    const u32x4 gq = prep_load(pp.qn, c, pp.style), gk = prep_load(pp.kn, c, pp.style);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < VECS; ++i) {
+      const int v = 4 * wave + r + 4 * S::WAVES * i, row = v / HEADS, hh = v % HEADS;
+      if (m0 + row >= p.M) continue;   // uniform over the 16-lane row
+      const int head = n0 / ATT_D + hh;
+      const bool isq = head < pp.Hq, normed = head < pp.Hq + pp.Hkv;
+      const u32x4 raw = prep_load(tile + row * LD + hh * ATT_D, c, pp.style);
+      const u32x4 y = prep_vector(raw, rp[i], isq ? gq : gk, normed, pp.style, pp.eps);
+      uint16_t* dst;
+      if (isq) dst = pp.q + (((size_t)bb[i] * pp.Hq + head) * pp.T + tt[i]) * ATT_D;
+      else if (normed) dst = pp.kc + (((size_t)bb[i] * pp.Hkv + (head - pp.Hq)) * pp.cap + pp.p0 + tt[i]) * ATT_D;
+      else dst = pp.vc + (((size_t)bb[i] * pp.Hkv + (head - pp.Hq - pp.Hkv)) * pp.cap + pp.p0 + tt[i]) * ATT_D;
+      prep_store(dst, c, pp.style, y);
     }
     return;
   }
@@ -555,7 +552,6 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   float* const s_ys = reinterpret_cast<float*>(smem);   // [BM][WN]
 #pragma unroll
   for (int mi = 0; mi < MS; ++mi) {
-    if (!stores) break;
     const int row0 = m0 + 16 * fr[mi] + 4 * r;
     if (!paired) {
       uint32_t res[4][NJ / 2];
@@ -614,15 +610,13 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
   if (p.ys) {
     // 64 output columns (128 of the tile's) are one half group of the next product's k
     constexpr int WH = 128 / (16 * NJ);   // waves a half group
-    if constexpr (BN % 128 == 0) {
-      __syncthreads();
-      for (int q = tid; q < BM * (BN / 128); q += S::THREADS) {
-        const int row = q % BM, h = q / BM;
-        float v = s_ys[row * WN + h * WH];
+    __syncthreads();
+    for (int q = tid; q < BM * (BN / 128); q += S::THREADS) {
+      const int row = q % BM, h = q / BM;
+      float v = s_ys[row * WN + h * WH];
 #pragma unroll
-        for (int w = 1; w < WH; ++w) v += s_ys[row * WN + h * WH + w];
-        if (m0 + row < p.M) p.ys[(size_t)((n0 >> 7) + h) * p.ldys + m0 + row] = v;
-      }
+      for (int w = 1; w < WH; ++w) v += s_ys[row * WN + h * WH + w];
+      if (m0 + row < p.M) p.ys[(size_t)((n0 >> 7) + h) * p.ldys + m0 + row] = v;
     }
   }
 }
@@ -632,31 +626,36 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
 namespace {
 using namespace t2i;
 
-template <int MF, int NJ, int WN, int WK>
+template <int MF, int NJ, int WN, int WK, bool GIVEN>
 hipError_t launch_one(const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
   using S = GemmShape<MF, NJ, WN, WK, 0>;
   const unsigned tiles = (unsigned)((p.M + S::BM - 1) / S::BM) * (unsigned)(p.N / S::BN);
-  if (!p.xs) hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 0>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
-  else if (p.xs_parts == 1) hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 1>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
-  else hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 2>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
+  if (!p.xs) {
+    hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 0>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
+  } else if constexpr (GIVEN) {
+    if (p.xs_parts == 1) hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 1>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
+    else hipLaunchKernelGGL((w4a16_prompt_kernel<MF, NJ, WN, WK, 2>), dim3(tiles), dim3(S::THREADS), 0, s, p, pp);
+  } else {
+    return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
 }  // namespace
 
-// Tile configurations: (row fragments a wave, columns a lane, waves along N, k slices).
+// Tile forms (PROMPT_FORMS of prompt_plan.h): row fragments a wave, columns a lane, waves along
+// N, k slices, and whether it is built for given row sums.
 #define T2I_PROMPT_CONFIGS(X) \
-  X(8, 2, 8, 1)               \
-  X(4, 2, 4, 1)               \
-  X(4, 2, 4, 2)               \
-  X(2, 2, 2, 4)
+  X(8, 2, 8, 1, true)         \
+  X(4, 2, 4, 1, false)        \
+  X(4, 2, 4, 2, true)
 
 namespace t2i_host {
 
 hipError_t launch_prompt_ring(const PromptPlan& pl, const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
-  if (!prompt_form_serves(pl, p.N, p.epi == EPI_QKV_PREP || p.xs || p.ys)) return hipErrorInvalidValue;
-#define T2I_PROMPT_LAUNCH(a, b, c, d) \
-  if (pl.cfg[0] == a && pl.cfg[1] == b && pl.cfg[2] == c && pl.cfg[3] == d) return launch_one<a, b, c, d>(p, pp, s);
+  if (!prompt_form_serves(pl, p.N, p.xs != nullptr)) return hipErrorInvalidValue;
+#define T2I_PROMPT_LAUNCH(a, b, c, d, given) \
+  if (pl.cfg[0] == a && pl.cfg[1] == b && pl.cfg[2] == c && pl.cfg[3] == d) return launch_one<a, b, c, d, given>(p, pp, s);
   T2I_PROMPT_CONFIGS(T2I_PROMPT_LAUNCH)
 #undef T2I_PROMPT_LAUNCH
   return hipErrorInvalidValue;

@@ -762,7 +762,7 @@ hipError_t launch_plan(const LinearPlan& pl, const LinearParams& p, bool norm, b
 // The prompt GEMM over p's rows, with its own row sums or p.xs in p.xs_parts parts.
 hipError_t launch_gemm(const PromptPlan& pl, const LinearParams& p, const QkvPrepParams& pp, hipStream_t s) {
   if (pl.kind == PromptPlan::RING) return t2i_host::launch_prompt_ring(pl, p, pp, s);
-  if (pl.kind != PromptPlan::TILES64 || !t2i_host::prompt_form_serves(pl, p.N, true)) return hipErrorInvalidValue;
+  if (pl.kind != PromptPlan::TILES64 || !t2i_host::prompt_form_serves(pl, p.N, p.xs != nullptr)) return hipErrorInvalidValue;
   const unsigned tiles = (unsigned)((p.M + GM_BM - 1) / GM_BM) * (unsigned)(p.N / GM_BN);
   if (!p.xs) hipLaunchKernelGGL(w4a16_gemm_kernel<0>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
   else if (p.xs_parts == 1) hipLaunchKernelGGL(w4a16_gemm_kernel<1>, dim3(tiles), dim3(GM_THREADS), 0, s, p, pp);
@@ -837,7 +837,7 @@ int run_linear(int epi, const uint16_t* x, int M, const uint16_t* gamma, float e
       return fail(T2I_ERR_ALIGN, "chained-norm buffers: 16-byte aligned (ss_out 4-byte)");
     if (M >= PROMPT_ROWS) return fail(T2I_ERR_SHAPE, "M=%d: the chained norm serves fewer than %d rows", M, PROMPT_ROWS);
   }
-  const PromptPlan prompt = gamma || chain ? PromptPlan{PromptPlan::NONE, {0, 0, 0, 0}} : plan_prompt(M, K, N);
+  const PromptPlan prompt = gamma || chain ? PromptPlan{PromptPlan::NONE, {0, 0, 0, 0}} : plan_prompt(M, K, N, xs && M >= PROMPT_ROWS);
   if (prompt.kind != PromptPlan::NONE && (M >= PROMPT_ROWS || (qweight && !ys))) {
     // the LDS-tiled GEMMs, over the AutoGPTQ words (without them, fewer rows than a prompt
     // batch's read the tiles below)
@@ -935,7 +935,7 @@ int run_prefill_qkv(const uint16_t* x, const float* x_sums, int32_t B, int32_t T
   p.xs = x_sums;
   p.xs_parts = 1;
   p.ldxs = p.M;
-  return t2i_host::hip_status(launch_gemm(plan_prompt(p.M, K, N), p, pp, reinterpret_cast<hipStream_t>(stream)), "prefill projection launch");
+  return t2i_host::hip_status(launch_gemm(plan_prompt(p.M, K, N, x_sums != nullptr), p, pp, reinterpret_cast<hipStream_t>(stream)), "prefill projection launch");
 }
 }  // namespace
 
