@@ -135,8 +135,12 @@ struct AttnParams {
   float eps, scale;
 };
 
-// More splits than this are merged by a kernel of their own (decode_attention_merge_kernel).
-constexpr int ATT_MERGE_CHAIN = 32;
+// More splits than this are merged by a kernel of their own (decode_attention_merge_kernel):
+// from 33 on while the (sequence, kv head) pairs are a CU's worth each or fewer, from 64 on with
+// more, whose chains run beside other pairs' chunks (512 pairs of 8 q heads, full caches, us with
+// the chain / with the kernel: 34 splits 120 / 131, 50 172 / 178, 64 216 / 219 and on short
+// positions 132 / 125, 100 334 / 329; 128 pairs of one, 34 splits: 52.6 / 48.9).
+constexpr int ATT_MERGE_CHAIN = 32, ATT_MERGE_CHAIN_FULL = 63, ATT_MERGE_FULL = 256;
 
 // One workgroup per (sequence b, kv head h, chunk of 16 * ROWS context slots).
 // A single workgroup per (b, h) streaming the whole context was measured 2-4x
@@ -165,7 +169,7 @@ constexpr int ATT_MERGE_CHAIN = 32;
 //   PREP = false (t2i_decode_attention_prepared): q, k and v come normalised and
 //   rotated already, as three row arrays: qkv_ = q [B, Hq*D], qn_ = k [B, Hkv*D],
 //   kn_ = v [B, Hkv*D]; no norm weights and no RoPE table are read.
-//   LONG: more than ATT_MERGE_CHAIN splits; the states are left to the merge kernel.
+//   LONG: more splits than a chain merges; the states are left to the merge kernel.
 template <int Q, int ROWS, bool PREP = true, bool LONG = false>
 __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const int32_t* pos_, const uint16_t* qkv_,
                                                                        uint16_t* kc_, uint16_t* vc_,
@@ -985,7 +989,7 @@ template <int Q, int ROWS, bool PREP>
 hipError_t launch_attention(const AttnParams& p, dim3 grid, hipStream_t s) {
   const int heads = p.Hq | p.Hkv << 15 | p.style << 30;
   const int cap_chunk = (int)((unsigned)p.ctx_cap | (unsigned)p.chunk << 23);
-  if (p.splits <= ATT_MERGE_CHAIN) {
+  if (p.splits <= (grid.x > ATT_MERGE_FULL ? ATT_MERGE_CHAIN_FULL : ATT_MERGE_CHAIN)) {
     hipLaunchKernelGGL((decode_attention_kernel<Q, ROWS, PREP>), grid, dim3(ATT_THREADS), 0, s, p.pos, p.qkv, p.kc,
                        p.vc, p.qn, p.kn, heads, cap_chunk, p);
     return hipGetLastError();
