@@ -118,16 +118,20 @@ __device__ __forceinline__ i32x4 tile_rsrc(const void* p) {
 }
 // One 16-byte (dma4: 4-byte) piece a lane into LDS at lds + 16 (4) lane, written as asm so
 // that the compiler's own waits (it waits for every load into LDS before any LDS read)
-// leave it in flight; dma_wait covers it.  M0 takes the LDS address, with one wait state
-// before the load.  lanes: all (~0) or none (0: nothing is read or written, and nothing is
-// assumed of when such a load counts or leaves the count: waits past one wait for everything);
-// every call is made by whole waves, so all lanes are on again after it.
+// leave it in flight; dma_wait covers it.  M0 takes the LDS address, with a wait state before
+// the load.  The compiler does not look into asm for hazards: an SGPR that a VALU instruction
+// wrote (a v_readfirstlane) is five wait states away from a VMEM instruction that reads it, and
+// the two moves and the s_nop are five whatever stands before them (without the s_nop, whose
+// place nothing the compiler emitted here needed, 0.2 to 0.5 % faster).  lanes: all (~0) or none
+// (0: nothing is read or written, and nothing is assumed of when such a load counts or leaves the
+// count: waits past one wait for everything); every call is made by whole waves, so all lanes
+// are on again after it.
 __device__ __forceinline__ void dma16(i32x4 rsrc, uint32_t off, uint32_t soff, uint32_t lds, uint64_t lanes) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b64 exec, -1"
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\ts_mov_b64 exec, -1"
                :: "s"(lds), "v"(off), "s"(rsrc), "s"(soff), "s"(lanes) : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(i32x4 rsrc, uint32_t off, uint32_t soff, uint32_t lds, uint64_t lanes) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %4\n\tbuffer_load_dword %1, %2, %3 offen lds\n\ts_mov_b64 exec, -1"
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %4\n\ts_nop 2\n\tbuffer_load_dword %1, %2, %3 offen lds\n\ts_mov_b64 exec, -1"
                :: "s"(lds), "v"(off), "s"(rsrc), "s"(soff), "s"(lanes) : "memory", "m0");
 }
 // Until at most N of this wave's vector memory operations are in flight.
