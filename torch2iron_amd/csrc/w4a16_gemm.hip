@@ -64,6 +64,7 @@ struct GemmShape {
   static constexpr int OPS_A = KSG, OPS_W = W_BYTES / 1024 / WN, OPS_S = (PIECES + WN - 1) / WN;
   static constexpr int OPS = OPS_A + OPS_S + OPS_W;
   static_assert(MF == WN && (MF & (MF - 1)) == 0 && MF % WK == 0, "a row fragment a wave, whole pieces");
+  static_assert(NJ == 2, "the epilogue stores a pair of columns a lane");
   static_assert(BN % 128 == 0 && ATT_D == 128, "whole heads and half groups of output sums a tile");
   static_assert(W_BYTES % (1024 * WN) == 0 && OPS_S <= 2, "the same number of loads in every wave");
 };
@@ -145,7 +146,7 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 }
 
 template <int MF, int NJ, int WN, int WK, int XSP>
-__global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1) void w4a16_prompt_kernel(const LinearParams p, const QkvPrepParams pp) {
+__global__ __launch_bounds__(64 * WN * WK, 2) void w4a16_prompt_kernel(const LinearParams p, const QkvPrepParams pp) {
   using S = GemmShape<MF, NJ, WN, WK, XSP>;
   constexpr int BM = S::BM, BN = S::BN;
   __shared__ __align__(16) unsigned char smem[S::LDS];
@@ -578,8 +579,7 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
         }
         if (row0 + i < p.M) {
           uint32_t* dst = reinterpret_cast<uint32_t*>(p.y0 + (size_t)(row0 + i) * p.ldy + ncol);
-          if constexpr (NJ == 4) *reinterpret_cast<u32x2*>(dst) = u32x2{v[0], v[1]};
-          else dst[0] = v[0];
+          dst[0] = v[0];
         }
       }
     } else {
@@ -596,13 +596,8 @@ __global__ __launch_bounds__(64 * WN * WK, WN * WK >= 8 || MF * NJ <= 16 ? 2 : 1
         }
         const size_t off = (size_t)(row0 + i) * p.ldy + (ncol >> 1);
         if (row0 + i < p.M) {
-          if constexpr (NJ == 4) {
-            *reinterpret_cast<uint32_t*>(p.y0 + off) = pack_bf16x2(o0[0], o0[1]);
-            if (p.epi == EPI_PAIRED) *reinterpret_cast<uint32_t*>(p.y1 + off) = pack_bf16x2(o1[0], o1[1]);
-          } else {
-            p.y0[off] = (uint16_t)f32_to_bf16(o0[0]);
-            if (p.epi == EPI_PAIRED) p.y1[off] = (uint16_t)f32_to_bf16(o1[0]);
-          }
+          p.y0[off] = (uint16_t)f32_to_bf16(o0[0]);
+          if (p.epi == EPI_PAIRED) p.y1[off] = (uint16_t)f32_to_bf16(o1[0]);
         }
         if (p.ys) {   // the wave's 8 NJ output columns of the row
           hs = row_sum16(hs);
