@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from oracle import w4a16 as ow
+from torch2iron_amd import _lib
 from torch2iron_amd import model as gm
 from torch2iron_amd import ops
 from torch2iron_amd.formats import W4A16Weight, interleave_gate_up
@@ -124,6 +125,25 @@ def test_swiglu_output_sums(gpu, m, k, n):
     assert torch.equal(h, ops.gate_up(x, w))
     hd = h.double().view(m, -1, 64)
     assert ((hs.double().t() - hd.sum(-1)).abs() <= 1e-5 * hd.abs().sum(-1) + 1e-30).all()
+
+
+@pytest.mark.parametrize("form,m,k,n", [s for s in SHAPES if s[1] < ops.PROMPT_GEMM_ROWS and s[2] >= 1024],
+                         ids=_ids([s for s in SHAPES if s[1] < ops.PROMPT_GEMM_ROWS and s[2] >= 1024]))
+def test_tiles_without_the_words(gpu, form, m, k, n):
+    """65 to 511 rows over the tiles alone (qweight NULL) run the decode kernel whatever the plan names:
+    the reference's value within the same bar, and the same bits as a call with both where the plan is
+    the decode tiles too."""
+    w, x = ops.tile_weight(_weight(k, n, m + k, gpu)), _x(m, k, m + n, gpu)
+    y = torch.empty(m, n, dtype=BF16, device=gpu)
+    rc = _lib.load().t2i_w4a16_linear_tiles(x.data_ptr(), m, None, 0.0, None, w.tiles.data_ptr(), w.qzeros.data_ptr(),
+                                            w.scales.data_ptr(), k, n, 128, _lib.T2I_TILES_STORE, None, y.data_ptr(),
+                                            None, _lib.stream_handle(gpu))
+    _lib.check(rc, "t2i_w4a16_linear_tiles")
+    ref = _ref(x, w)
+    assert ((y.double() - ref).abs() <= _bound(ref)).all()
+    both = ops.linear(x, w)
+    assert ((both.double() - ref).abs() <= _bound(ref)).all()
+    assert form != "decode tiles" or torch.equal(y, both)
 
 
 @pytest.mark.parametrize("style", [0, 1])

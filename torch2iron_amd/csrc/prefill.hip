@@ -310,12 +310,16 @@ __device__ __forceinline__ float row4_max(float v) {
 
 // The same product with two sets of 16 query rows a wave (128 rows a workgroup).  With one
 // set a wave reads the whole K and V block (32 KB) for 16 rows: 1024 cycles of LDS a block
-// for a workgroup against 512 of MFMA.  With two, every read feeds two MFMAs and the
-// softmax (16 exponentials a lane, set and block, at a quarter rate) bounds it.  Two block
+// for a workgroup against 512 of MFMA.  With two, every read feeds two MFMAs.  Two block
 // buffers (one barrier a block), two workgroups a CU; each lane sums its own keys' weights
 // and the four sums of a row meet after the last block; the outputs are rescaled only when a
-// row of the wave has a new max.  1999 rows from 6001 on, 32 q / 8 kv heads: 398 -> 300 us
-// (764 TFLOP/s); 16 x 250 rows from 500 on: 88 -> 71 us; 16 x 512 from 0, 16 / 8: 47.8 -> 44 us.
+// row of the wave has a new max.  What bounds it: no unit alone.  Over 1999 rows from 6001 on, 32
+// q / 8 kv heads, VALU instructions (the softmax, its exponentials and packing) take 50 % of the
+// SIMDs' cycles, MFMAs 33 %, LDS reads 41 % of the CUs', and waves wait for a third of their time;
+// over 16 x 512 rows from 0 (36, 17 and 21 %) 28 % of the CUs' time is before and after the
+// blocks: launch, the first q, K and V loads, the outputs.  us with one set a wave -> two: 1999
+// rows 386 -> 278 (823 TFLOP/s); 16 x 250 rows from 500 on, 16 / 8: 45.4 -> 35.5; 16 x 512 rows
+// 42.0 -> 39.7.
 template <int Q>
 __global__ __launch_bounds__(256, 2) void prefill_attention_wide_kernel(const PrefillAttnParams p) {
   constexpr int D = PF_D;

@@ -14,7 +14,7 @@ namespace t2i_host {
 // on, 1 to 500 sequences, 1, 2, 4 and 8 q heads a kv head, graph-launched):
 //   n1, n2    blocks of 64 and of 128 rows.  A block of 128 costs 1.47 of 64 in the long run,
 //             so padding decides short chunks (64 x 20 rows from 500, 8 kv heads of 2: as many
-//             blocks either way, 128-row ones a quarter slower);
+//             blocks either way, 25.6 us with 64 rows and 31.3 with 128);
 //   even, k   n2 in blocks of the longest one's length (a block's work grows from p0 to p0 + T
 //             keys: with few of them the longest block is the call), and a block's mean 64-key
 //             blocks (under 1.5 what a workgroup starts with outweighs its products);
@@ -24,9 +24,9 @@ namespace t2i_host {
 //             of the longest one's length on (0.999 to 1.69 times there).
 // Of those calls it sends 870 to the 128-row blocks: 7 are 2 to 8 % slower than with 64-row
 // ones, the rest 0.98 to 1.72 times as fast, the median 1.22.  (us, 64-row / 128-row: 1999 rows
-// from 6001, 32 / 8 heads 385 / 279; 16 x 512 rows from 0, 16 / 8: 43 / 41; and kept with 64-row
-// blocks: 312 x 1 row from 0, 8 / 8 12.0 / 19.7, 56 x 129 rows from 0, 8 / 8 18.6 / 22.5, 2000
-// rows from 0, 16 / 8 53 / 61.)
+// from 6001, 32 / 8 heads 386 / 278; 16 x 250 rows from 500, 16 / 8: 45.4 / 35.5; 16 x 512 rows
+// from 0, 16 / 8: 42.0 / 39.7; and kept with 64-row blocks: 312 x 1 row from 0, 8 / 8 12.0 /
+// 19.7, 56 x 129 rows from 0, 8 / 8 18.6 / 22.5, 2000 rows from 0, 16 / 8 49.3 / 58.5.)
 inline bool prefill_wide(int B, int T, int p0, int Hkv, int Q) {
   const double heads = (double)B * Hkv, last = (double)p0 + T, mean = p0 + 0.5 * T;
   const double n1 = heads * ((T + 64 / Q - 1) / (64 / Q)), n2 = heads * ((T + 128 / Q - 1) / (128 / Q));

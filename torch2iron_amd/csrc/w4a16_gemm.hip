@@ -21,17 +21,18 @@
 //   * Step s + 1's words are unpacked beside step s's MFMAs, the previous fragment's sums
 //     are folded beside the next one's, loads go out one every few MFMAs.  The order is the
 //     program's (empty asm ties; the compiler otherwise sinks the folds and unpacking behind
-//     the MFMAs and spills: 256 registers and scratch against 222 and none).
+//     the MFMAs and spills: 256 registers and scratch against 225 and none).
 //   * The two waves of a SIMD step down in priority through a step, so the one that is
 //     behind goes first; without it the older one runs ahead and waits at the step's barrier
-//     while the other runs alone (497 -> 470 us at 8192 x 2048 x 12288).
-// What bounds it: at 128 x 256 each of 8 waves reads all 128 rows' fragments, 2800 cycles of
-// LDS reads a step against 2176 of MFMA and about 2300 of VALU and MFMA issue; a step takes
-// about 4000.  Wider waves (64 columns) read half as much but need more than 256 registers:
-// one wave a SIMD then, measured slower (536 us).  Against the 64 x 128 kernel (us, M x K x N,
-// graph-launched): gate_up 8192 x 2048 x 12288 620 -> 455, down 4001 x 6144 x 2048 150 -> 105,
-// 8192 x 2048 x 4096 197 -> 144, 8192 x 1024 x 4096 100 -> 86; against the decode tiles, gate_up
-// 331 x 2048 x 12288 55 -> 33.
+//     while the other runs alone (497 -> 470 us at 8192 x 2048 x 12288 when it was added).
+// What bounds it: instruction issue.  At 8192 x 2048 x 12288 (128 x 256 tiles) MFMAs take 44 % of
+// the SIMDs' cycles and VALU instructions 39 % beside them (unpacking, folding); the LDS index
+// unit is busy for 32 % of the CUs' cycles and waves wait to issue to it for 4 % of theirs.  A short
+// K adds the prologue and the epilogue of its one workgroup a CU: at K = 1024 MFMAs take 28 to 34
+// %.  Wider waves (64 columns) need more than 256 registers: one wave a SIMD then, measured slower
+// (536 us).  Against the 64 x 128 kernel (us, M x K x N, graph-launched in turn): gate_up 8192 x
+// 2048 x 12288 584 -> 438, down 4001 x 6144 x 2048 146 -> 103, 8192 x 2048 x 4096 190 -> 164, 8192
+// x 1024 x 4096 107 -> 104; against the decode tiles, gate_up 331 x 2048 x 12288 52 -> 33.
 #include <type_traits>
 
 #include "t2i_common.h"

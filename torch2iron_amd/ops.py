@@ -16,7 +16,7 @@ from torch2iron_amd.formats import GROUP_SIZE, W4A16Weight
 BF16 = torch.bfloat16
 
 ROPE_HALVES = 0
-PROMPT_GEMM_ROWS = 512   # rows from which the linear always runs a prompt GEMM (65 to 511: where it is faster)
+PROMPT_GEMM_ROWS = 512   # rows from which outputs of whole 128 columns run a prompt GEMM (65 to 511: where it is faster)
 ROPE_INTERLEAVED = 1
 
 
