@@ -7,7 +7,7 @@ library next to this file.  The library exports the C ABI of
 ``python -m torch2iron_amd.build --tuning PATH`` writes a second library to PATH
 with ``T2I_TUNING`` defined: its plan functions then honour the environment
 overrides ``T2I_PLAN`` and ``T2I_RT`` (decode linear tile plan and row-tile
-height), ``T2I_PROMPT`` (form of the prompt GEMM: row fragments, columns a lane, waves, k
+height), ``T2I_XROWS_MIN_RT`` (smallest row tile given whole-row loads), ``T2I_PROMPT`` (form of the prompt GEMM: row fragments, columns a lane, waves, k
 slices, or anything else for the 64 x 128 kernel) and
 ``T2I_ATTN_ROWS`` (decode attention rows per chunk), for sweeps of the launch
 shapes.  Swap it in place of ``libt2i_hip.so`` to use it.

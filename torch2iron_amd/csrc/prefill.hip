@@ -314,10 +314,10 @@ __device__ __forceinline__ float row4_max(float v) {
 // buffers (one barrier a block), two workgroups a CU; each lane sums its own keys' weights
 // and the four sums of a row meet after the last block; the outputs are rescaled only when a
 // row of the wave has a new max.  What bounds it: no unit alone.  Over 1999 rows from 6001 on, 32
-// q / 8 kv heads, VALU instructions (the softmax, its exponentials and packing) take 50 % of the
-// SIMDs' cycles, MFMAs 33 %, LDS reads 41 % of the CUs', and waves wait for a third of their time;
-// over 16 x 512 rows from 0 (36, 17 and 21 %) 28 % of the CUs' time is before and after the
-// blocks: launch, the first q, K and V loads, the outputs.  us with one set a wave -> two: 1999
+// q / 8 kv heads, VALU instructions (the softmax, its exponentials and packing) take 47 % of the
+// cycles of a SIMD that holds waves, MFMAs 38 % and LDS reads 47 % of the CU's, and waves wait for
+// a third of their time; over 16 x 512 rows from 0 it is 44, 23 and 29 %: a workgroup has eight
+// blocks at most, and its first loads and its outputs lie open.  us with one set a wave -> two: 1999
 // rows 386 -> 278 (823 TFLOP/s); 16 x 250 rows from 500 on, 16 / 8: 45.4 -> 35.5; 16 x 512 rows
 // 42.0 -> 39.7.
 template <int Q>

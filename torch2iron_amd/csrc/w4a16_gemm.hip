@@ -25,11 +25,11 @@
 //   * The two waves of a SIMD step down in priority through a step, so the one that is
 //     behind goes first; without it the older one runs ahead and waits at the step's barrier
 //     while the other runs alone (497 -> 470 us at 8192 x 2048 x 12288 when it was added).
-// What bounds it: instruction issue.  At 8192 x 2048 x 12288 (128 x 256 tiles) MFMAs take 44 % of
-// the SIMDs' cycles and VALU instructions 39 % beside them (unpacking, folding); the LDS index
-// unit is busy for 32 % of the CUs' cycles and waves wait to issue to it for 4 % of theirs.  A short
-// K adds the prologue and the epilogue of its one workgroup a CU: at K = 1024 MFMAs take 28 to 34
-// %.  Wider waves (64 columns) need more than 256 registers: one wave a SIMD then, measured slower
+// What bounds it: instruction issue.  At 8192 x 2048 x 12288 (128 x 256 tiles) MFMAs take 47 % of
+// the cycles of a SIMD that holds waves and VALU instructions 42 % beside them (unpacking,
+// folding); the LDS index unit is busy for 35 % and waves wait to issue to it for 4 % of theirs.  A
+// short K adds the prologue and the epilogue of its one workgroup a CU: MFMAs 32 % of the fused
+// q|k|v projection at K = 1024.  Wider waves (64 columns) need more than 256 registers: one wave a SIMD then, measured slower
 // (536 us).  Against the 64 x 128 kernel (us, M x K x N, graph-launched in turn): gate_up 8192 x
 // 2048 x 12288 584 -> 438, down 4001 x 6144 x 2048 146 -> 103, 8192 x 2048 x 4096 190 -> 164, 8192
 // x 1024 x 4096 107 -> 104; against the decode tiles, gate_up 331 x 2048 x 12288 52 -> 33.
